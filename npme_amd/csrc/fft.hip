@@ -1,4 +1,4 @@
-// Batched 1-D Stockham FFT passes in LDS for gfx950.
+// Batched 1-D FFT passes in LDS for gfx950.
 //
 // The reciprocal-sum convolution theta = IDFT(G . DFT(Q)) is computed on the
 // zero-padded full grid (N1 x N2 x N3) but only the compact quarter-volume
@@ -13,14 +13,29 @@
 // exist.  The twiddle table holds exp(-2 pi i t/N) computed in FP64 on the
 // host.
 //
-// A workgroup of 256 threads transforms B columns (B a power of two) held in
-// LDS; every thread owns one column and a strided subset of its butterflies,
-// so all per-column index arithmetic is done once, with shifts.  Strided
-// passes keep LDS as [n][c] (B consecutive columns side by side: global rows
-// of B complex values, 128 B for B = 16 in FP32, map to contiguous LDS);
-// row passes keep [c][n] with one element of padding per column.  Between
-// the read and the write barrier of a stage every thread holds its
-// butterflies in registers, so one LDS buffer suffices.
+// General lengths (7-smooth, even): a Stockham transform of 2 to 4 stages
+// with radices up to 16 (make_plan), every stage a switch over compile-time
+// butterflies.  A thread owns whole butterflies of one column.  The first
+// stage reads global memory straight into its butterflies and the last one
+// writes global memory from them, so LDS carries only the exchanges between
+// stages (one for two stages, two for three); in the convolution the last
+// forward stage, the k-space multiply and the first backward stage are one
+// step in registers: the backward transform runs the radices in reverse
+// order, so its first butterflies take the rows that the forward transform's
+// last ones produced.  Between the read and the write barrier of a stage a
+// thread holds its butterflies in registers, so one LDS buffer suffices.
+//
+// What bounds it: HBM (each pass reads and writes its data once), provided
+// enough loads are in flight; the LDS round trips and barriers of a stage
+// are the rest, so fewer and larger radices pay.  The earlier form (radices
+// 8/4/2/7/5/3, a separate LDS fill, LDS drain and G pass, ~170 VGPRs, 4096
+// values a workgroup whatever the length, so 2 to 4 adjacent columns at
+// lengths near 1000) took, FP32, passes A/B/C/D/E: 32/60/96/56/31 us on 256 x
+// 384 x 500 (now 24/34/58/37/25: 4.4 TB/s in B), 79/124/558/119/77 on 320 x
+// 320 x 1152 (now 50/92/212/91/60), 42/85/342/80/41 on 448^3 (now
+// 37/68/157/68/45); FP64 120^3 15/14/23/13/14 (now 10/10/14/10/9).
+// N = 64 and 512 have kernels of their own (below) with every index a
+// compile-time constant.
 #include <type_traits>
 
 #include "npme_internal.h"
@@ -68,11 +83,17 @@ __device__ __forceinline__ double load_or_zero(const double *p, long idx, bool o
   return ok ? x : 0.0;
 }
 
-constexpr int NT = 256;  // threads per workgroup
+constexpr int NT = 256;  // threads per workgroup of the 8^L kernels
 
+// stages of a general plan: radices in forward order; for the forward (F)
+// and the reversed (B) order the twiddle stride N / (Ns R) of each stage and
+// the multiplier M = ceil(2^22 / Ns) with which j mod Ns is j - ((j M) >> 22)
+// Ns (exact for j Ns < 2^22: j and Ns are below 2^11)
 struct PlanDev {
   int N, nst;
-  int radix[24];
+  int radix[4];
+  int strF[4], strB[4];
+  unsigned magF[4], magB[4];
 };
 
 // ------------------------------------------------------------ small DFTs
@@ -189,101 +210,396 @@ template <typename T, int R> struct DFTOdd {
   }
 };
 
+
+// cos and sin of 2 pi a / b at compile time (|angle| reduced below pi / 4
+// by symmetry is not needed: 24 Taylor terms give FP64 accuracy to |x| <= pi)
+constexpr double ct_pi = 3.14159265358979323846;
+constexpr double ct_cos(int a, int b)
+{
+  a %= b;
+  if (2 * a > b) a -= b;
+  const double x = 2 * ct_pi * a / b;
+  double s = 0, t = 1;
+  for (int k = 0; k < 24; k++) {
+    s += t;
+    t *= -x * x / ((2 * k + 1) * (2 * k + 2));
+  }
+  return s;
+}
+constexpr double ct_sin(int a, int b)
+{
+  a %= b;
+  if (2 * a > b) a -= b;
+  const double x = 2 * ct_pi * a / b;
+  double s = 0, t = x;
+  for (int k = 0; k < 24; k++) {
+    s += t;
+    t *= -x * x / ((2 * k + 2) * (2 * k + 3));
+  }
+  return s;
+}
+
+template <typename T, int R> __device__ __forceinline__ void dft_any(T *x);
+
+// R = A B with coprime factors (Good-Thomas): x[(B a + A b) mod R] is a 2-D
+// A x B array, X[k] its 2-D transform at (k mod A, k mod B); no twiddles
+template <typename T, int A, int B> __device__ __forceinline__ void dft_coprime(T *x)
+{
+  constexpr int R = A * B;
+  T y[B][A];
+#pragma unroll
+  for (int b = 0; b < B; b++) {
+#pragma unroll
+    for (int a = 0; a < A; a++) y[b][a] = x[(B * a + A * b) % R];
+    dft_any<T, A>(y[b]);
+  }
+#pragma unroll
+  for (int a = 0; a < A; a++) {
+    T z[B];
+#pragma unroll
+    for (int b = 0; b < B; b++) z[b] = y[b][a];
+    dft_any<T, B>(z);
+#pragma unroll
+    for (int b = 0; b < B; b++) y[b][a] = z[b];
+  }
+#pragma unroll
+  for (int k = 0; k < R; k++) x[k] = y[k % B][k % A];
+}
+
+template <int R, int I> struct TwConst {
+  static constexpr double c = ct_cos(I, R), s = ct_sin(I, R);
+};
+// x * exp(-2 pi i I / R)
+template <typename T, int R, int I> __device__ __forceinline__ T mul_root(T x)
+{
+  using S = decltype(T::x);
+  if constexpr (I % R == 0) return x;
+  else if constexpr (4 * (I % R) == R) return mul_mi(x);
+  else {
+    constexpr S c = (S)TwConst<R, I>::c, s = (S)TwConst<R, I>::s;
+    return mk<T>(x.x * c + x.y * s, x.y * c - x.x * s);
+  }
+}
+template <typename T, int A, int K, int B0> __device__ __forceinline__ void root_row(T *y)
+{
+  // y[k] *= exp(-2 pi i k B0 / (A A)), k = K .. A-1
+  if constexpr (K < A) {
+    y[K] = mul_root<T, A * A, K * B0>(y[K]);
+    root_row<T, A, K + 1, B0>(y);
+  }
+}
+template <typename T, int A, int B0> __device__ __forceinline__ void square_rows(const T *x, T (*y)[A])
+{
+  if constexpr (B0 < A) {
+#pragma unroll
+    for (int a = 0; a < A; a++) y[B0][a] = x[A * a + B0];
+    dft_any<T, A>(y[B0]);
+    root_row<T, A, 1, B0>(y[B0]);
+    square_rows<T, A, B0 + 1>(x, y);
+  }
+}
+// R = A^2 (9, 16): Cooley-Tukey with compile-time twiddles
+template <typename T, int A> __device__ __forceinline__ void dft_square(T *x)
+{
+  T y[A][A];
+  square_rows<T, A, 0>(x, y);
+#pragma unroll
+  for (int k1 = 0; k1 < A; k1++) {
+    T z[A];
+#pragma unroll
+    for (int b = 0; b < A; b++) z[b] = y[b][k1];
+    dft_any<T, A>(z);
+#pragma unroll
+    for (int k2 = 0; k2 < A; k2++) x[k1 + A * k2] = z[k2];
+  }
+}
+
 template <typename T, int R> __device__ __forceinline__ void dft_any(T *x)
 {
-  if constexpr (R == 5 || R == 7)
-    DFTOdd<T, R>::run(x);
-  else
-    DFT<T, R>::run(x);
+  if constexpr (R == 5 || R == 7) DFTOdd<T, R>::run(x);
+  else if constexpr (R == 6) dft_coprime<T, 2, 3>(x);
+  else if constexpr (R == 10) dft_coprime<T, 2, 5>(x);
+  else if constexpr (R == 12) dft_coprime<T, 4, 3>(x);
+  else if constexpr (R == 9) dft_square<T, 3>(x);
+  else if constexpr (R == 16) dft_square<T, 4>(x);
+  else DFT<T, R>::run(x);
 }
 
-// ------------------------------------------------------------ column access
-// element n of the thread's column: [c][n] (row layout, stride ld = N + 1)
-// or [n][c] (strided layout, B columns side by side)
-struct ColRef {
-  int base, sh;  // lds index = base + n * 2^sh (the step is 1 or the column count)
+// ------------------------------------------------------------ general stages
+// a thread's place: column c of the workgroup, the tj-th of tpc threads of
+// that column; row n of the column sits at base + (n << sh) in LDS.  The
+// first exchange (written by a first stage of radix R: rows j R + r) leaves
+// one row free after every R, so neighbouring threads' writes spread over
+// the banks: row n at n + n / R, which stays linear in r for the writer
+// (j (R + 1) + r) and for the reader (j + r nb, nb a multiple of R).
+struct Place {
+  int c, tj, tpc;
+  int base, sh;
   __device__ __forceinline__ int at(int n) const { return base + (n << sh); }
 };
-
-// ------------------------------------------------------------ Stockham stage
-// butterfly j of a column reads x[j + r N/R], twiddles by w^(r k N/(Ns R)),
-// k = j mod Ns, and writes y[(j - k) R + k + r Ns].  POW2: N and Ns are
-// powers of two, so the modulo is a mask (the generic form divides).
-template <typename T, int R, int BPT, bool POW2>
-__device__ __forceinline__ void stage(T *lds, ColRef col, int tj, int tpc, int N, int Ns,
-                                      const T *__restrict__ tw)
+// rows of a column in LDS: N, and the free rows of the first exchange in
+// either direction
+__host__ __device__ inline int column_rows(const PlanDev &p)
 {
-  const int nb = N / R;
-  const int stride = N / (Ns * R);
-  T v[BPT][R];
-#pragma unroll
-  for (int u = 0; u < BPT; u++) {
-    const int j = tj + u * tpc;
-    if (j < nb) {
-#pragma unroll
-      for (int r = 0; r < R; r++) v[u][r] = lds[col.at(j + r * nb)];
-    }
+  const int a = p.radix[0], b = p.radix[p.nst - 1];
+  return p.N + p.N / (a < b ? a : b);
+}
+
+// strided layout: B = 2^lgB columns side by side
+__device__ __forceinline__ Place place_cols(int lgB)
+{
+  Place p;
+  p.c = threadIdx.x & ((1 << lgB) - 1);
+  p.tj = threadIdx.x >> lgB;
+  p.tpc = blockDim.x >> lgB;
+  p.base = p.c;
+  p.sh = lgB;
+  return p;
+}
+// row layout: C columns one after another, tpc threads each; the threads
+// past C tpc have no butterfly
+__device__ __forceinline__ Place place_rows(int C, int tpc, int rows)
+{
+  Place p;
+  p.c = threadIdx.x / tpc;
+  p.tj = threadIdx.x - p.c * tpc;
+  if (p.c >= C) {
+    p.c = 0;
+    p.tj = 1 << 24;
   }
-  __syncthreads();
-#pragma unroll
-  for (int u = 0; u < BPT; u++) {
-    const int j = tj + u * tpc;
-    if (j < nb) {
-      const int k = (Ns == 1) ? 0 : (POW2 ? (j & (Ns - 1)) : j % Ns);
-      if (k != 0) {
-#pragma unroll
-        for (int r = 1; r < R; r++) v[u][r] = cmul(v[u][r], tw[r * k * stride]);
+  p.tpc = tpc;
+  p.base = p.c * rows;
+  p.sh = 0;
+  return p;
+}
+
+// butterflies of radix R that one thread holds at a time: up to MV values or
+// one butterfly.  With MV >= 14 a column of at most 4095 values needs at most
+// 512 threads.
+constexpr int bpt_of(int R, int MV) { return R > MV ? 1 : MV / R; }
+// columns in FP32: two radix-8 butterflies (fewer, busier threads: pass C at
+// 448 points 194 -> 156 us, 280^3 complex 107 -> 82 us against one); in FP64
+// two would need more than 128 VGPRs (512-point pass C 434 -> 516 us), and
+// row passes are slower with two as well
+template <typename Real, bool ROWS> constexpr int hold() { return sizeof(Real) == 4 && !ROWS ? 16 : 14; }
+
+// one call of f(integral_constant<int, R>) for the plan's radix
+template <bool EVEN, typename F> __device__ __forceinline__ void with_radix(int R, F &&f)
+{
+  switch (R) {
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 10: f(std::integral_constant<int, 10>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    case 16: f(std::integral_constant<int, 16>{}); break;
+    default:
+      if constexpr (!EVEN) {
+        switch (R) {
+          case 3: f(std::integral_constant<int, 3>{}); break;
+          case 5: f(std::integral_constant<int, 5>{}); break;
+          case 7: f(std::integral_constant<int, 7>{}); break;
+          case 9: f(std::integral_constant<int, 9>{}); break;
+          default: break;
+        }
       }
-      dft_any<T, R>(v[u]);
-      const int idx = (j - k) * R + k;
-#pragma unroll
-      for (int r = 0; r < R; r++) lds[col.at(idx + r * Ns)] = v[u][r];
-    }
+      break;
   }
+}
+
+// first stage (Ns = 1): butterfly j takes the elements get(j, r nb), that
+// is rows j + r nb with nb = N/R, and writes rows j R + r (with the free
+// rows).  HALF: the elements from N/2 on are zero and not read (R is even
+// then).  get runs for every slot (butterfly 0 in place of those past the
+// last), so no load sits behind a per-lane branch and a thread's loads are
+// all in flight together.  INLDS: get reads this column from LDS.
+template <typename T, int MV, bool HALF, bool INLDS, typename G>
+__device__ __forceinline__ void stage_first(T *lds, const Place &p, int N, int R0, G &&get)
+{
+  with_radix<HALF>(R0, [&](auto rc) {
+    constexpr int R = decltype(rc)::value, BPT = bpt_of(R, MV);
+    const int nb = N / R;
+    T v[BPT][R];
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc, jj = j < nb ? j : 0;
+#pragma unroll
+      for (int r = 0; r < R; r++) v[u][r] = (HALF && r >= R / 2) ? mk<T>(0, 0) : get(jj, r * nb);
+    }
+    if constexpr (INLDS) __syncthreads();
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc;
+      if (j < nb) {
+        dft_any<T, R>(v[u]);
+        T *w = lds + p.at(j * (R + 1));
+#pragma unroll
+        for (int r = 0; r < R; r++) w[r << p.sh] = v[u][r];
+      }
+    }
+  });
   __syncthreads();
 }
 
-// radix classes of a plan: the kernels are compiled for the radices a plan
-// can contain, since every stage variant in the switch adds registers
-// (radix 8 only: ~80 VGPRs, 8/4/2: ~110, all six: ~170)
-enum { RC_ALL = 0, RC_POW2 = 1, RC_R8 = 2 };
-
-// all stages of the plan on every column of the workgroup; EMAX bounds the
-// elements one thread holds (N / tpc <= EMAX)
-template <typename T, int EMAX, int RC>
-__device__ void fft_columns(T *lds, ColRef col, int tj, int tpc, const PlanDev &p,
-                            const T *__restrict__ tw)
+// inner stage: reads x[j + r nb], nb = N/R, twiddles by w^(r k N/(Ns R)), k
+// = j mod Ns, writes y[(j - k) R + k + r Ns]; in LDS, in place.  gap: the
+// rows read are those of the first exchange (a free row after every Ns)
+template <typename T, int MV>
+__device__ __forceinline__ void stage_inner(T *lds, const Place &p, int N, int Rs, int Ns, int str,
+                                            unsigned mag, bool gap, const T *tw)
 {
-  constexpr bool P2 = RC != RC_ALL;
-  int Ns = 1;
-  for (int s = 0; s < p.nst; s++) {
-    const int R = p.radix[s];
-    switch (R) {
-      case 8: stage<T, 8, (EMAX + 7) / 8, P2>(lds, col, tj, tpc, p.N, Ns, tw); break;
-      case 4:
-        if constexpr (RC != RC_R8) stage<T, 4, (EMAX + 3) / 4, P2>(lds, col, tj, tpc, p.N, Ns, tw);
-        break;
-      case 2:
-        if constexpr (RC != RC_R8) stage<T, 2, (EMAX + 1) / 2, P2>(lds, col, tj, tpc, p.N, Ns, tw);
-        break;
-      case 3:
-        if constexpr (RC == RC_ALL) stage<T, 3, (EMAX + 2) / 3, P2>(lds, col, tj, tpc, p.N, Ns, tw);
-        break;
-      case 5:
-        if constexpr (RC == RC_ALL) stage<T, 5, (EMAX + 4) / 5, P2>(lds, col, tj, tpc, p.N, Ns, tw);
-        break;
-      case 7:
-        if constexpr (RC == RC_ALL) stage<T, 7, (EMAX + 6) / 7, P2>(lds, col, tj, tpc, p.N, Ns, tw);
-        break;
-      default: break;
+  with_radix<false>(Rs, [&](auto rc) {
+    constexpr int R = decltype(rc)::value, BPT = bpt_of(R, MV);
+    const int nb = N / R;
+    const int step = (gap ? nb + nb / Ns : nb) << p.sh;
+    T v[BPT][R];
+    int q[BPT];  // j / Ns
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc;
+      q[u] = (int)(((unsigned)j * mag) >> 22);
+      if (j < nb) {
+        const T *x = lds + p.at(gap ? j + q[u] : j);
+#pragma unroll
+        for (int r = 0; r < R; r++) v[u][r] = x[r * step];
+      }
     }
-    Ns *= R;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc;
+      if (j < nb) {
+        const int qN = q[u] * Ns, k = j - qN;
+        const T *t = tw;
+        const int ks = k * str;
+#pragma unroll
+        for (int r = 1; r < R; r++) {
+          t += ks;
+          v[u][r] = cmul(v[u][r], *t);
+        }
+        dft_any<T, R>(v[u]);
+        T *y = lds + p.at(qN * R + k);
+#pragma unroll
+        for (int r = 0; r < R; r++) y[r * Ns << p.sh] = v[u][r];
+      }
+    }
+  });
+  __syncthreads();
+}
+
+// rows j + r nb of a last stage (Ns = nb) into v; gap: two-stage plans read
+// the first exchange, whose free rows come after every nb
+template <typename T, int R>
+__device__ __forceinline__ void last_read(const T *lds, const Place &p, int j, int nb, bool gap, T *v)
+{
+  const T *x = lds + p.at(j);
+  const int step = (gap ? nb + 1 : nb) << p.sh;
+#pragma unroll
+  for (int r = 0; r < R; r++) v[r] = x[r * step];
+}
+template <typename T, int R> __device__ __forceinline__ void last_dft(const T *tw, int j, T *v)
+{
+  const T *t = tw;
+#pragma unroll
+  for (int r = 1; r < R; r++) {
+    t += j;
+    v[r] = cmul(v[r], *t);
+  }
+  dft_any<T, R>(v);
+}
+
+// last stage (Ns = N/R, so k = j): put(j, r, r nb, value) receives row j + r
+// nb.  TOLDS: put writes this column in LDS
+template <typename T, int MV, bool TOLDS, typename P>
+__device__ __forceinline__ void stage_last(T *lds, const Place &p, int N, int Rs, bool gap, const T *tw, P &&put)
+{
+  with_radix<false>(Rs, [&](auto rc) {
+    constexpr int R = decltype(rc)::value, BPT = bpt_of(R, MV);
+    const int nb = N / R;
+    T v[BPT][R];
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc;
+      if (j < nb) last_read<T, R>(lds, p, j, nb, gap, v[u]);
+    }
+    if constexpr (TOLDS) __syncthreads();
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc;
+      if (j < nb) {
+        last_dft<T, R>(tw, j, v[u]);
+#pragma unroll
+        for (int r = 0; r < R; r++) put(j, r, r * nb, v[u][r]);
+      }
+    }
+  });
+}
+
+// last forward stage, f(g, value) on its rows with g = pre(j, r nb) (a load
+// issued before the stage), first backward stage of the same radix: rows j +
+// r N/R in, j R + r (with the free rows) out
+template <typename T, int MV, typename GT, typename L, typename F>
+__device__ __forceinline__ void stage_turn(T *lds, const Place &p, int N, int Rs, bool gap, const T *tw, L &&pre,
+                                           F &&f)
+{
+  with_radix<false>(Rs, [&](auto rc) {
+    constexpr int R = decltype(rc)::value, BPT = bpt_of(R, MV);
+    const int nb = N / R;
+    T v[BPT][R];
+    GT g[BPT][R];
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc, jj = j < nb ? j : 0;
+#pragma unroll
+      for (int r = 0; r < R; r++) g[u][r] = pre(jj, r * nb);
+    }
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc;
+      if (j < nb) last_read<T, R>(lds, p, j, nb, gap, v[u]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < BPT; u++) {
+      const int j = p.tj + u * p.tpc;
+      if (j < nb) {
+        last_dft<T, R>(tw, j, v[u]);
+#pragma unroll
+        for (int r = 0; r < R; r++) v[u][r] = f(g[u][r], v[u][r]);
+        dft_any<T, R>(v[u]);
+        T *w = lds + p.at(j * (R + 1));
+#pragma unroll
+        for (int r = 0; r < R; r++) w[r << p.sh] = v[u][r];
+      }
+    }
+  });
+  __syncthreads();
+}
+
+// the inner stages of a transform, in forward or reversed radix order
+template <typename T, int MV>
+__device__ __forceinline__ void stages_inner(T *lds, const Place &p, const PlanDev &pl, bool rev, const T *tw)
+{
+  int Ns = pl.radix[rev ? pl.nst - 1 : 0];
+  for (int s = 1; s < pl.nst - 1; s++) {
+    const int i = rev ? pl.nst - 1 - s : s;
+    stage_inner<T, MV>(lds, p, pl.N, pl.radix[i], Ns, rev ? pl.strB[s] : pl.strF[s],
+                rev ? pl.magB[s] : pl.magF[s], s == 1, tw);
+    Ns *= pl.radix[i];
   }
 }
 
-// at most 4096 complex values (32 KB FP32, 64 KB FP64) per workgroup, so
-// several workgroups share a CU and overlap their load, LDS and store phases
-template <typename Real> constexpr int emax() { return 16; }
+// the twiddle table, copied into LDS behind the columns (a butterfly reads
+// R - 1 of them; from LDS rather than a global load each); ordered by the
+// barrier that ends the first stage
+template <typename T>
+__device__ __forceinline__ const T *twiddles_in(T *lds, int ldsElems, int N, const T *tw)
+{
+  T *tl = lds + ldsElems;
+  for (int i = threadIdx.x; i < N; i += blockDim.x) tl[i] = tw[i];
+  return tl;
+}
 
 // workgroups are dealt round-robin to the 8 XCDs; remap so each XCD walks a
 // contiguous range of columns (adjacent column groups share L2 lines)
@@ -292,75 +608,6 @@ __device__ __forceinline__ int xcd_wg()
   const int wg = blockIdx.x, nwg = gridDim.x;
   const int x = wg & 7, local = wg >> 3, q = nwg >> 3, r = nwg & 7;
   return x * q + min(x, r) + local;
-}
-
-// thread -> (column, index within column) for the two layouts
-struct Lane {
-  int c, tj, tpc;
-  ColRef col;
-};
-__device__ __forceinline__ Lane lane_strided(int lgB, int N)
-{
-  Lane L;
-  const int B = 1 << lgB;
-  L.c = threadIdx.x & (B - 1);
-  L.tj = threadIdx.x >> lgB;
-  L.tpc = NT >> lgB;
-  L.col.base = L.c;
-  L.col.sh = lgB;
-  (void)N;
-  return L;
-}
-__device__ __forceinline__ Lane lane_rows(int lgB, int N)
-{
-  Lane L;
-  L.tpc = NT >> lgB;
-  L.c = threadIdx.x >> (8 - lgB);  // NT = 2^8
-  L.tj = threadIdx.x & (L.tpc - 1);
-  L.col.base = L.c * (N + 1);
-  L.col.sh = 0;
-  return L;
-}
-
-// loads of one column into LDS: all of a thread's (at most EMAX) elements
-// are fetched into registers first, so its global loads are in flight
-// together, then stored; get(n) returns element n (n < N) with no branch
-// around its loads
-template <typename T, int EMAX, typename F>
-__device__ __forceinline__ void stage_in(T *lds, const Lane &L, int N, F &&get)
-{
-  T v[EMAX];
-  // get runs for every slot (element 0 in place of those past N), so no
-  // load sits behind a per-lane branch
-#pragma unroll
-  for (int u = 0; u < EMAX; u++) {
-    const int n = L.tj + u * L.tpc;
-    v[u] = get(n < N ? n : 0);
-  }
-#pragma unroll
-  for (int u = 0; u < EMAX; u++) {
-    const int n = L.tj + u * L.tpc;
-    if (n < N) lds[L.col.at(n)] = v[u];
-  }
-}
-
-// twiddle table of the pass: copied into LDS behind the column data in FP32
-// (data <= 32 KB plus N <= 4096 entries stay within 64 KB; FP64 columns
-// already fill 64 KB), so the butterflies read it with ds_read instead of a
-// global load per twiddled element; the copy is ordered by the barrier that
-// follows stage_in
-template <typename Real> constexpr bool twl_lds() { return sizeof(Real) == 4; }
-
-template <typename T, bool TWL>
-__device__ __forceinline__ const T *twiddles_in(T *lds, int ldsElems, int N, const T *tw)
-{
-  if constexpr (TWL) {
-    T *tl = lds + ldsElems;
-    for (int i = threadIdx.x; i < N; i += NT) tl[i] = tw[i];
-    return tl;
-  } else {
-    return tw;
-  }
 }
 
 // ------------------------------------------------------------ pass kernels
@@ -372,66 +619,113 @@ struct CGeom {
   int inOuter, inInner, inPos, outOuter, outInner, outPos;
 };
 
-template <typename Real, bool ROWS, int RC>
-__global__ __launch_bounds__(NT) void k_fft_complex(CGeom g, PlanDev p, const typename Cx<Real>::T *tw,
-                                                    const typename Cx<Real>::T *__restrict__ in,
-                                                    typename Cx<Real>::T *__restrict__ out, int lgB,
-                                                    int backward)
+// threads of a workgroup at most (FP64 butterflies need twice the registers)
+template <typename Real> constexpr int max_threads() { return sizeof(Real) == 4 ? 1024 : 512; }
+
+// strided columns (passes B and D): HIN: only the first N/2 elements are
+// non-zero.  rev: the radices in reversed order (the first radix of a plan
+// is even, the end at which half the elements are missing: the start of pass
+// B, the finish of pass D)
+template <typename Real, bool HIN>
+__global__ __launch_bounds__(max_threads<Real>()) void k_fft_cols(CGeom g, PlanDev pl,
+                                                                  const typename Cx<Real>::T *tw,
+                                                                  const typename Cx<Real>::T *__restrict__ in,
+                                                                  typename Cx<Real>::T *__restrict__ out,
+                                                                  int lgB, int backward)
 {
   using T = typename Cx<Real>::T;
+  constexpr int MV = hold<Real, false>();
   extern __shared__ char smem_raw[];
   T *lds = reinterpret_cast<T *>(smem_raw);
   const int N = g.N;
-  const Lane L = ROWS ? lane_rows(lgB, N) : lane_strided(lgB, N);
-  const int colg = (xcd_wg() << lgB) + L.c;
+  const Place p = place_cols(lgB);
+  const int colg = (xcd_wg() << lgB) + p.c;
   const int o0 = colg / g.nInner;
   const bool valid = colg < g.nCols && colg - o0 * g.nInner < g.validInner;
   const int o = valid ? o0 : 0, i = valid ? colg - o0 * g.nInner : 0;
   const T *src = in + ((long)o * g.inOuter + (long)i * g.inInner);
-  const T *twl = twiddles_in<T, twl_lds<Real>()>(lds, (1 << lgB) * (ROWS ? N + 1 : N), N, tw);
-  stage_in<T, emax<Real>()>(lds, L, N, [&](int n) {
-    const T v = load_or_zero(src, (long)n * g.inPos, valid && n < g.Lin);
-    return backward ? cconj(v) : v;
+  const T *twl = twiddles_in(lds, column_rows(pl) << lgB, N, tw);
+  const bool rev = backward;
+  // an invalid column reads column 0 and is not stored
+  stage_first<T, MV, HIN, false>(lds, p, N, pl.radix[rev ? pl.nst - 1 : 0], [&](int j, int rnb) {
+    T x;
+    if constexpr (HIN) x = (src + (long)j * g.inPos)[(long)rnb * g.inPos];
+    else x = load_or_zero(src, (long)(j + rnb) * g.inPos, j + rnb < g.Lin);
+    return backward ? cconj(x) : x;
   });
-  __syncthreads();
-  fft_columns<T, emax<Real>(), RC>(lds, L.col, L.tj, L.tpc, p, twl);
-  if (!valid) return;
+  stages_inner<T, MV>(lds, p, pl, rev, twl);
   T *dst = out + ((long)o * g.outOuter + (long)i * g.outInner);
-  for (int n = L.tj; n < g.Lout; n += L.tpc) {
-    T v = lds[L.col.at(n)];
-    if (backward) v = cconj(v);
-    dst[(long)n * g.outPos] = v;
-  }
+  stage_last<T, MV, false>(lds, p, N, pl.radix[rev ? 0 : pl.nst - 1], pl.nst == 2, twl,
+                       [&](int j, int r, int rnb, T v) {
+    if (valid && j + rnb < g.Lout) (dst + (long)j * g.outPos)[(long)rnb * g.outPos] = backward ? cconj(v) : v;
+  });
 }
 
-// pass A: two real rows per complex column, R2C by the two-for-one split
-template <typename Real, int RC>
-__global__ __launch_bounds__(NT) void k_fft_r2c(int N, int Lin, int nPairs, int inRow, int outRow,
-                                                PlanDev p, const typename Cx<Real>::T *tw,
-                                                const Real *__restrict__ in,
-                                                typename Cx<Real>::T *__restrict__ out, int lgB)
+// contiguous rows (passes A and E of complex charges): C rows a workgroup
+template <typename Real, bool HIN>
+__global__ __launch_bounds__(max_threads<Real>()) void k_fft_rows(CGeom g, PlanDev pl,
+                                                                  const typename Cx<Real>::T *tw,
+                                                                  const typename Cx<Real>::T *__restrict__ in,
+                                                                  typename Cx<Real>::T *__restrict__ out, int C,
+                                                                  int tpc, int backward)
 {
   using T = typename Cx<Real>::T;
+  constexpr int MV = hold<Real, true>();
   extern __shared__ char smem_raw[];
   T *lds = reinterpret_cast<T *>(smem_raw);
-  const Lane L = lane_rows(lgB, N);
-  const int pr = (xcd_wg() << lgB) + L.c;
-  const bool valid = pr < nPairs;
-  const Real *ra = in + (valid ? (long)(2 * pr) * inRow : 0), *rb = ra + (valid ? inRow : 0);
-  const T *twl = twiddles_in<T, twl_lds<Real>()>(lds, (1 << lgB) * (N + 1), N, tw);
-  stage_in<T, emax<Real>()>(lds, L, N, [&](int n) {
-    const bool ok = valid && n < Lin;
-    return mk<T>(load_or_zero(ra, n, ok), load_or_zero(rb, n, ok));
+  const int N = g.N;
+  const Place p = place_rows(C, tpc, column_rows(pl));
+  const int row = xcd_wg() * C + p.c;
+  const bool valid = row < g.nCols;
+  const int i = valid ? row : 0;
+  const T *src = in + (long)i * g.inInner;
+  T *dst = out + (long)i * g.outInner;
+  const T *twl = twiddles_in(lds, C * column_rows(pl), N, tw);
+  const bool rev = backward;
+  stage_first<T, MV, HIN, false>(lds, p, N, pl.radix[rev ? pl.nst - 1 : 0], [&](int j, int rnb) {
+    T x;
+    if constexpr (HIN) x = (src + j)[rnb];
+    else x = load_or_zero(src, j + rnb, j + rnb < g.Lin);
+    return backward ? cconj(x) : x;
   });
+  stages_inner<T, MV>(lds, p, pl, rev, twl);
+  stage_last<T, MV, false>(lds, p, N, pl.radix[rev ? 0 : pl.nst - 1], pl.nst == 2, twl,
+                       [&](int j, int r, int rnb, T v) {
+    if (valid && j + rnb < g.Lout) (dst + j)[rnb] = backward ? cconj(v) : v;
+  });
+}
+
+// pass A: two real rows per complex row, R2C by the two-for-one split (Lin
+// = N/2 data values a row)
+template <typename Real>
+__global__ __launch_bounds__(max_threads<Real>()) void k_fft_r2c(int nPairs, int inRow, int outRow,
+                                                                 PlanDev pl, const typename Cx<Real>::T *tw,
+                                                                 const Real *__restrict__ in,
+                                                                 typename Cx<Real>::T *__restrict__ out, int C,
+                                                                 int tpc)
+{
+  using T = typename Cx<Real>::T;
+  constexpr int MV = hold<Real, true>();
+  extern __shared__ char smem_raw[];
+  T *lds = reinterpret_cast<T *>(smem_raw);
+  const int N = pl.N;
+  const Place p = place_rows(C, tpc, column_rows(pl));
+  const int pr = xcd_wg() * C + p.c;
+  const bool valid = pr < nPairs;
+  const Real *ra = in + (valid ? (long)(2 * pr) * inRow : 0), *rb = ra + inRow;
+  const T *twl = twiddles_in(lds, C * column_rows(pl), N, tw);
+  stage_first<T, MV, true, false>(lds, p, N, pl.radix[0],
+                              [&](int j, int rnb) { return mk<T>((ra + j)[rnb], (rb + j)[rnb]); });
+  stages_inner<T, MV>(lds, p, pl, false, twl);
+  stage_last<T, MV, true>(lds, p, N, pl.radix[pl.nst - 1], pl.nst == 2, twl,
+                      [&](int j, int r, int rnb, T v) { (lds + p.at(j))[rnb] = v; });
   __syncthreads();
-  fft_columns<T, emax<Real>(), RC>(lds, L.col, L.tj, L.tpc, p, twl);
   if (!valid) return;
-  const int K = N / 2 + 1;
   const Real h = (Real)0.5;
   T *oa = out + (long)(2 * pr) * outRow, *ob = oa + outRow;
-  for (int k = L.tj; k < K; k += L.tpc) {
-    const T z = lds[L.col.at(k)];
-    const T w = cconj(lds[L.col.at(k == 0 ? 0 : N - k)]);
+  for (int k = p.tj; k <= N / 2; k += tpc) {
+    const T z = lds[p.at(k)];
+    const T w = cconj(lds[p.at(k == 0 ? 0 : N - k)]);
     const T s = cadd(z, w), d = csub(z, w);
     oa[k] = mk<T>(h * s.x, h * s.y);
     ob[k] = mk<T>(h * d.y, -h * d.x);  // -i d / 2
@@ -439,57 +733,55 @@ __global__ __launch_bounds__(NT) void k_fft_r2c(int N, int Lin, int nPairs, int 
 }
 
 // pass E: Hermitian half rows -> two real rows (backward transform)
-template <typename Real, int RC>
-__global__ __launch_bounds__(NT) void k_fft_c2r(int N, int Lout, int nPairs, int inRow, int outRow,
-                                                PlanDev p, const typename Cx<Real>::T *tw,
-                                                const typename Cx<Real>::T *__restrict__ in,
-                                                Real *__restrict__ out, int lgB)
+template <typename Real>
+__global__ __launch_bounds__(max_threads<Real>()) void k_fft_c2r(int Lout, int nPairs, int inRow, int outRow,
+                                                                 PlanDev pl, const typename Cx<Real>::T *tw,
+                                                                 const typename Cx<Real>::T *__restrict__ in,
+                                                                 Real *__restrict__ out, int C, int tpc)
 {
   using T = typename Cx<Real>::T;
+  constexpr int MV = hold<Real, true>();
   extern __shared__ char smem_raw[];
   T *lds = reinterpret_cast<T *>(smem_raw);
-  const Lane L = lane_rows(lgB, N);
-  const int pr = (xcd_wg() << lgB) + L.c;
+  const int N = pl.N, h = N / 2;
+  const Place p = place_rows(C, tpc, column_rows(pl));
+  const int pr = xcd_wg() * C + p.c;
   const bool valid = pr < nPairs;
-  const int h = N / 2;
-  const T *ia = in + (valid ? (long)(2 * pr) * inRow : 0), *ib = ia + (valid ? inRow : 0);
-  const T *twl = twiddles_in<T, twl_lds<Real>()>(lds, (1 << lgB) * (N + 1), N, tw);
-  {
-    // each stored element m = 0 .. N/2 of the two Hermitian rows is loaded
-    // once and gives both rows n = m and n = N - m of the column:
-    // Z = Xa + i Xb (n <= N/2), conj(Xa) + i conj(Xb) above; stored conj(Z).
-    // The thread's loads are all issued (index clamped, no branch around
-    // them) before the LDS stores; nu, the slots a thread needs, is uniform
-    constexpr int EH = emax<Real>() / 2 + 1;
-    const int nu = (h + L.tpc) / L.tpc;
-    T a[EH], b[EH];
+  const T *ia = in + (valid ? (long)(2 * pr) * inRow : 0), *ib = ia + inRow;
+  const T *twl = twiddles_in(lds, C * column_rows(pl), N, tw);
+  // each stored element m = 0 .. N/2 of the two Hermitian rows is loaded
+  // once and gives both elements n = m and n = N - m of the column:
+  // Z = Xa + i Xb (n <= N/2), conj(Xa) + i conj(Xb) above; stored conj(Z).
+  // Four elements' loads are in flight together.
+  for (int m0 = p.tj; m0 <= h; m0 += 4 * tpc) {
+    T a[4], b[4];
 #pragma unroll
-    for (int u = 0; u < EH; u++) {
-      if (u < nu) {
-        const int m = L.tj + u * L.tpc;
-        const bool ok = valid && m <= h;
-        a[u] = load_or_zero(ia, m <= h ? m : 0, ok);
-        b[u] = load_or_zero(ib, m <= h ? m : 0, ok);
-      }
+    for (int u = 0; u < 4; u++) {
+      const int m = m0 + u * tpc;
+      a[u] = ia[m <= h ? m : 0];
+      b[u] = ib[m <= h ? m : 0];
     }
 #pragma unroll
-    for (int u = 0; u < EH; u++) {
-      const int m = L.tj + u * L.tpc;
-      if (u < nu && m <= h) {
-        lds[L.col.at(m)] = mk<T>(a[u].x - b[u].y, -(a[u].y + b[u].x));
-        if (m > 0 && m < h) lds[L.col.at(N - m)] = mk<T>(a[u].x + b[u].y, a[u].y - b[u].x);
+    for (int u = 0; u < 4; u++) {
+      const int m = m0 + u * tpc;
+      if (m <= h) {
+        lds[p.at(m)] = mk<T>(a[u].x - b[u].y, -(a[u].y + b[u].x));
+        if (m > 0 && m < h) lds[p.at(N - m)] = mk<T>(a[u].x + b[u].y, a[u].y - b[u].x);
       }
     }
   }
   __syncthreads();
-  fft_columns<T, emax<Real>(), RC>(lds, L.col, L.tj, L.tpc, p, twl);
-  if (!valid) return;
+  // reversed radix order: the stage that writes half its elements is the
+  // last one
+  stage_first<T, MV, false, true>(lds, p, N, pl.radix[pl.nst - 1], [&](int j, int rnb) { return (lds + p.at(j))[rnb]; });
+  stages_inner<T, MV>(lds, p, pl, true, twl);
   Real *oa = out + (long)(2 * pr) * outRow, *ob = oa + outRow;
-  for (int n = L.tj; n < Lout; n += L.tpc) {
-    const T z = lds[L.col.at(n)];  // conj of the backward transform
-    oa[n] = z.x;
-    ob[n] = -z.y;
-  }
+  stage_last<T, MV, false>(lds, p, N, pl.radix[0], pl.nst == 2, twl, [&](int j, int r, int rnb, T z) {
+    if (valid && j + rnb < Lout) {
+      (oa + j)[rnb] = z.x;  // z: conj of the backward transform
+      (ob + j)[rnb] = -z.y;
+    }
+  });
 }
 
 // G of pass C.  GM 0: real G at (|k1|, |k2|, k3); GM 1: complex G at
@@ -530,56 +822,48 @@ template <int GM> __device__ __forceinline__ int g_a1(int n, int N, int gfl)
   else return (n <= N / 2) ? n : N - n;
 }
 
-// pass C: forward along axis 1, X <- X G, backward, keep the first Lin
-// outputs.  Columns c = k2 * C3 + k3.
-template <typename Real, int GM, int RC>
-__global__ __launch_bounds__(NT) void k_fft_conv(int N, int Lin, int nCols, int pos, int N2, int gfl,
-                                                 int C3, int Kv, int N3fold, PlanDev p,
-                                                 const typename Cx<Real>::T *tw, const void *Gv,
-                                                 typename Cx<Real>::T *__restrict__ data, int lgB)
+// pass C: forward along axis 1 (Lin = N/2 rows of data), X <- X G, backward,
+// keep the first N/2 outputs.  Columns c = k2 * C3 + k3.
+template <typename Real, int GM>
+__global__ __launch_bounds__(max_threads<Real>()) void k_fft_conv(int nCols, int pos, int N2, int gfl, int C3,
+                                                                  int Kv, int N3fold, PlanDev pl,
+                                                                  const typename Cx<Real>::T *tw, const void *Gv,
+                                                                  typename Cx<Real>::T *__restrict__ data, int lgB)
 {
   constexpr bool CG = GM > 0;
   using T = typename Cx<Real>::T;
+  using GT = typename std::conditional<CG, T, Real>::type;
+  constexpr int MV = hold<Real, false>();
   extern __shared__ char smem_raw[];
   T *lds = reinterpret_cast<T *>(smem_raw);
-  const Lane L = lane_strided(lgB, N);
-  const int colg = (xcd_wg() << lgB) + L.c;
+  const int N = pl.N;
+  const Place p = place_cols(lgB);
+  const int colg = (xcd_wg() << lgB) + p.c;
   // C3: row length of the data (padded); Kv: valid entries of a row
   const bool valid = colg < nCols && colg % C3 < Kv;
   T *col = data + (valid ? colg : 0);
-  const T *twl = twiddles_in<T, twl_lds<Real>()>(lds, (1 << lgB) * N, N, tw);
-  stage_in<T, emax<Real>()>(lds, L, N, [&](int n) {
-    return load_or_zero(col, (long)n * pos, valid && n < Lin);
-  });
-  __syncthreads();
-  fft_columns<T, emax<Real>(), RC>(lds, L.col, L.tj, L.tpc, p, twl);
-  // multiply by G and conjugate (for the backward transform)
+  const T *twl = twiddles_in(lds, column_rows(pl) << lgB, N, tw);
   const GIndex gi = g_index<GM>(N, N2, Kv, N3fold, gfl, valid, colg, C3);
-  constexpr int E = emax<Real>();
-  using GT = typename std::conditional<CG, T, Real>::type;
-  GT gv[E];
-#pragma unroll
-  for (int u = 0; u < E; u++) {  // the G loads of the thread, in flight together
-    const int n = L.tj + u * L.tpc;
-    const int nn = n < N ? n : 0;  // unconditional load (the value past N is unused)
-    gv[u] = reinterpret_cast<const GT *>(Gv)[(long)g_a1<GM>(nn, N, gfl) * 8 + gi.base];
+  const GT *Gp = reinterpret_cast<const GT *>(Gv) + gi.base;
+  // an invalid column reads column 0 and is not stored
+  stage_first<T, MV, true, false>(lds, p, N, pl.radix[0],
+                              [&](int j, int rnb) { return (col + (long)j * pos)[(long)rnb * pos]; });
+  stages_inner<T, MV>(lds, p, pl, false, twl);
+  // times G, conjugated for the backward transform
+  auto load_g = [&](int j, int rnb) {
+    GT gv = Gp[g_a1<GM>(j + rnb, N, gfl) * 8];
     if constexpr (GM == 2)
-      if (gfl & 8) gv[u] = cconj(gv[u]);
-  }
-#pragma unroll
-  for (int u = 0; u < E; u++) {
-    const int n = L.tj + u * L.tpc;
-    if (n < N) {
-      T x = lds[L.col.at(n)];
-      if constexpr (CG) x = cconj(cmul(x, gv[u]));
-      else x = mk<T>(gv[u] * x.x, -gv[u] * x.y);
-      lds[L.col.at(n)] = x;
-    }
-  }
-  __syncthreads();
-  fft_columns<T, emax<Real>(), RC>(lds, L.col, L.tj, L.tpc, p, twl);
-  if (!valid) return;
-  for (int n = L.tj; n < Lin; n += L.tpc) col[(long)n * pos] = cconj(lds[L.col.at(n)]);
+      if (gfl & 8) gv = cconj(gv);
+    return gv;
+  };
+  stage_turn<T, MV, GT>(lds, p, N, pl.radix[pl.nst - 1], pl.nst == 2, twl, load_g, [&](GT gv, T x) {
+    if constexpr (CG) return cconj(cmul(x, gv));
+    else return mk<T>(gv * x.x, -gv * x.y);
+  });
+  stages_inner<T, MV>(lds, p, pl, true, twl);
+  stage_last<T, MV, false>(lds, p, N, pl.radix[0], pl.nst == 2, twl, [&](int j, int r, int rnb, T v) {
+    if (valid && j + rnb < N / 2) (col + (long)j * pos)[(long)rnb * pos] = cconj(v);
+  });
 }
 
 // ------------------------------------------------------------ N = 8^L passes
@@ -614,6 +898,14 @@ template <typename T> __device__ __forceinline__ void dft8_half(T *x)
   x[6] = csub(e2, t2);
   x[3] = cadd(e3, t3);
   x[7] = csub(e3, t3);
+}
+
+// the twiddle table: in LDS behind the columns in FP32 (FP64 columns fill 64
+// KB and read it from global memory)
+template <typename T> __device__ __forceinline__ const T *twiddles8(T *lds, int ldsElems, int N, const T *tw)
+{
+  if constexpr (sizeof(T) == 8) return twiddles_in(lds, ldsElems, N, tw);
+  else return tw;
 }
 
 template <int L> struct P8 {
@@ -732,7 +1024,7 @@ __global__ __launch_bounds__(NT) void k_fft8_cols(CGeom g, const typename Cx<Rea
   const int o0 = colg / g.nInner;
   const bool valid = colg < g.nCols && colg - o0 * g.nInner < g.validInner;
   const int o = valid ? o0 : 0, i = valid ? colg - o0 * g.nInner : 0;
-  const T *twl = twiddles_in<T, twl_lds<Real>()>(lds, lds_elems8<T, L>(), P::N, tw);
+  const T *twl = twiddles8<T>(lds, lds_elems8<T, L>(), P::N, tw);
   const T *src = in + ((long)o * g.inOuter + (long)i * g.inInner);
   T v[P::BPT][8];
 #pragma unroll
@@ -786,7 +1078,7 @@ __global__ __launch_bounds__(NT) void k_fft8_conv(int nCols, int pos, int N2, in
   const int colg = (xcd_wg() << P::LGB) + c;
   const bool valid = colg < nCols && colg % C3 < Kv;
   T *col = data + (valid ? colg : 0);
-  const T *twl = twiddles_in<T, twl_lds<Real>()>(lds, lds_elems8<T, L>(), N, tw);
+  const T *twl = twiddles8<T>(lds, lds_elems8<T, L>(), N, tw);
   // the G values of the thread's rows, fetched up front
   const GIndex gi = g_index<GM>(N, N2, Kv, N3fold, gfl, valid, colg, C3);
   using GT = typename std::conditional<CG, T, Real>::type;
@@ -829,130 +1121,151 @@ __global__ __launch_bounds__(NT) void k_fft8_conv(int nCols, int pos, int N2, in
 }
 
 // set-up: even extension of a compact line (length N/2+1) to length N,
-// forward DFT, folded back to the compact line, in place (FP64)
-__global__ __launch_bounds__(NT) void k_fft_even(int N, int nCols, int nInner, int outer, int inner,
-                                                 int pos, PlanDev p, const double2 *tw,
-                                                 double2 *__restrict__ data, int lgB)
+// forward DFT, folded back to the compact line, in place (FP64).  PAIR: real
+// lines 2c and 2c + 1 share one complex transform z = a + i b; the transform
+// of a real even line is real, so A = Re Z and B = Im Z.
+template <bool PAIR>
+__global__ __launch_bounds__(max_threads<double>()) void k_fft_even(int nCols, int nInner, int outer, int inner,
+                                                                    int pos, PlanDev pl, const double2 *tw,
+                                                                    void *__restrict__ data, int lgB)
 {
+  using E = typename std::conditional<PAIR, double, double2>::type;
+  constexpr int MV = hold<double, false>();
   extern __shared__ char smem_raw[];
   double2 *lds = reinterpret_cast<double2 *>(smem_raw);
-  const int h = N / 2;
-  const Lane L = lane_strided(lgB, N);
-  const int colg = (xcd_wg() << lgB) + L.c;
-  const bool valid = colg < nCols;
-  const int o = valid ? colg / nInner : 0, i = valid ? colg - o * nInner : 0;
-  double2 *line = data + ((long)o * outer + (long)i * inner);
-  stage_in<double2, 16>(lds, L, N, [&](int n) {
-    return valid ? line[(long)((n <= h) ? n : N - n) * pos] : mk<double2>(0, 0);
-  });
-  __syncthreads();
-  fft_columns<double2, 16, RC_ALL>(lds, L.col, L.tj, L.tpc, p, tw);
-  if (!valid) return;
-  for (int n = L.tj; n <= h; n += L.tpc) {
-    double2 v = lds[L.col.at(n)];
-    if (n != 0 && n != h) {
-      const double2 w = lds[L.col.at(N - n)];
-      v = mk<double2>(0.5 * (v.x + w.x), 0.5 * (v.y + w.y));
-    }
-    line[(long)n * pos] = v;
-  }
-}
-
-// set-up, real even lines (the kernels 1/r and r^alpha): lines 2c and
-// 2c + 1 of a pass share one complex transform z = a + i b.  The transform
-// of a real even line is real, so A = Re Z and B = Im Z; folded back to the
-// compact line as in k_fft_even, in place (FP64)
-__global__ __launch_bounds__(NT) void k_fft_even_pair(int N, int nCols, int nInner, int outer,
-                                                      int inner, int pos, PlanDev p,
-                                                      const double2 *tw, double *__restrict__ data,
-                                                      int lgB)
-{
-  extern __shared__ char smem_raw[];
-  double2 *lds = reinterpret_cast<double2 *>(smem_raw);
-  const int h = N / 2;
-  const Lane L = lane_strided(lgB, N);
-  const int pair = (xcd_wg() << lgB) + L.c;
-  const int ca = 2 * pair, cb = 2 * pair + 1;
-  const bool va = ca < nCols, vb = cb < nCols;
+  const int N = pl.N, h = N / 2;
+  const Place p = place_cols(lgB);
+  const int cg = (xcd_wg() << lgB) + p.c;
+  const int ca = PAIR ? 2 * cg : cg, cb = ca + 1;
+  const bool va = ca < nCols, vb = PAIR && cb < nCols;
   auto line_of = [&](int c) {
     const int o = c / nInner, i = c - o * nInner;
-    return data + ((long)o * outer + (long)i * inner);
+    return static_cast<E *>(data) + ((long)o * outer + (long)i * inner);
   };
-  double *la = line_of(va ? ca : 0), *lb = line_of(vb ? cb : 0);
-  stage_in<double2, 16>(lds, L, N, [&](int n) {
+  E *la = line_of(va ? ca : 0), *lb = line_of(vb ? cb : 0);
+  const double2 *twl = twiddles_in(lds, column_rows(pl) << lgB, N, tw);
+  stage_first<double2, MV, false, false>(lds, p, N, pl.radix[0], [&](int j, int rnb) {
+    const int n = j + rnb;
     const long k = (long)((n <= h) ? n : N - n) * pos;
-    return mk<double2>(va ? la[k] : 0.0, vb ? lb[k] : 0.0);
+    // without a second line: zero, not line 0, which its own workgroup is
+    // rewriting (a changing b is not even, and would show in Re Z)
+    if constexpr (PAIR) {
+      const double b = lb[k];
+      return mk<double2>(la[k], vb ? b : 0.0);
+    }
+    else return la[k];
   });
+  stages_inner<double2, MV>(lds, p, pl, false, twl);
+  stage_last<double2, MV, true>(lds, p, N, pl.radix[pl.nst - 1], pl.nst == 2, twl,
+                            [&](int j, int r, int rnb, double2 v) { (lds + p.at(j))[rnb << p.sh] = v; });
   __syncthreads();
-  fft_columns<double2, 16, RC_ALL>(lds, L.col, L.tj, L.tpc, p, tw);
   if (!va) return;
-  for (int n = L.tj; n <= h; n += L.tpc) {
-    double2 v = lds[L.col.at(n)];
+  for (int n = p.tj; n <= h; n += p.tpc) {
+    double2 v = lds[p.at(n)];
     if (n != 0 && n != h) {
-      const double2 w = lds[L.col.at(N - n)];
+      const double2 w = lds[p.at(N - n)];
       v = mk<double2>(0.5 * (v.x + w.x), 0.5 * (v.y + w.y));
     }
-    la[(long)n * pos] = v.x;
-    if (vb) lb[(long)n * pos] = v.y;
+    if constexpr (PAIR) {
+      la[(long)n * pos] = v.x;
+      if (vb) lb[(long)n * pos] = v.y;
+    } else {
+      la[(long)n * pos] = v;
+    }
   }
 }
 
 // ------------------------------------------------------------ host side
 static PlanDev to_dev(const FFTPlan1D &p)
 {
-  PlanDev d;
+  if (p.nst < 2 || p.nst > 4) throw Error{NPME_ERR_GRID, "FFT length without a plan"};
+  PlanDev d{};
   d.N = p.N;
   d.nst = p.nst;
-  for (int i = 0; i < 24; i++) d.radix[i] = p.radix[i];
+  for (int i = 0; i < p.nst; i++) d.radix[i] = p.radix[i];
+  for (int rev = 0; rev < 2; rev++) {
+    int Ns = 1;
+    for (int s = 0; s < p.nst; s++) {
+      const int R = p.radix[rev ? p.nst - 1 - s : s];
+      (rev ? d.strB : d.strF)[s] = p.N / (Ns * R);
+      (rev ? d.magB : d.magF)[s] = ((1u << 22) + Ns - 1) / Ns;
+      Ns *= R;
+    }
+  }
   return d;
 }
 
-// columns per workgroup: a power of two with B * N <= EMAX * NT (strided
-// layout) or B * (N + 1) <= EMAX * NT (row layout), at most 64
-static int lg_batch(int N, bool fp64, bool rows)
+// threads a column needs: every stage's N / R butterflies in bpt_of(R)
+// rounds
+static int threads_per_column(const FFTPlan1D &p, int MV)
 {
-  const int cap = 16 * NT;
-  (void)fp64;
-  const int per = rows ? N + 1 : N;
-  int lg = 0;
-  while (lg < 6 && (2 << lg) * per <= cap) lg++;
-  return lg;
+  int t = 1;
+  for (int i = 0; i < p.nst; i++) {
+    const int nb = p.N / p.radix[i], b = bpt_of(p.radix[i], MV);
+    t = std::max(t, (nb + b - 1) / b);
+  }
+  return t;
 }
 
-static size_t lds_bytes(int N, int lgB, bool fp64, bool rows)
+struct FftLaunch {
+  int lgB, C, tpc, T;  // columns a workgroup (2^lgB strided, C rows), threads a column, threads
+  size_t lds;
+};
+
+// LDS of a workgroup: half a CU's 160 KB, so that two share a CU (long
+// columns: all of it)
+constexpr size_t kFftLds = 80 * 1024, kFftLdsMax = 160 * 1024;
+// a launch should have this many workgroups (four for each of 256 CUs)
+// before workgroups are made wider
+constexpr long kFftWide = 1024;
+
+// strided columns: 16 adjacent columns for short lengths where there are
+// enough of them, else 8 (64 bytes of FP32 complex values a row, half a cache
+// line; 8 and 4 in FP64), fewer only where LDS or the threads of a workgroup
+// do not allow them
+static FftLaunch launch_cols(const FFTPlan1D &p, bool fp64, long nCols)
 {
-  return (size_t)(1 << lgB) * (rows ? N + 1 : N) * (fp64 ? 16 : 8);
+  const int es = fp64 ? 16 : 8, maxT = fp64 ? 512 : 1024;
+  const int MV = fp64 ? hold<double, false>() : hold<float, false>();
+  const int tmin = threads_per_column(p, MV), rows = column_rows(to_dev(p));
+  const int lgMin = fp64 ? 2 : 3;
+  for (int lgB = lgMin + (p.N <= 256 && nCols >= (kFftWide << (lgMin + 1)) ? 1 : 0); lgB >= 0; lgB--) {
+    FftLaunch c{};
+    c.lgB = lgB;
+    const int B = 1 << lgB;
+    c.T = (B * tmin + 63) / 64 * 64;
+    c.tpc = c.T / B;
+    c.lds = ((size_t)rows * B + p.N) * es;
+    if (c.T <= maxT && c.lds <= (lgB > 0 ? kFftLds : kFftLdsMax)) return c;
+  }
+  throw Error{NPME_ERR_UNSUPPORTED, "FFT length " + std::to_string(p.N) + " does not fit a workgroup"};
 }
 
-// LDS of a pass: the columns, plus the twiddle table in FP32
-static size_t pass_lds(int N, int lgB, bool fp64, bool rows)
+// contiguous rows: about 256 threads a workgroup, fewer where the rows would
+// not give enough workgroups
+static FftLaunch launch_rows(const FFTPlan1D &p, bool fp64, long nRows)
 {
-  return lds_bytes(N, lgB, fp64, rows) + (fp64 ? 0 : (size_t)N * 8);
+  const int es = fp64 ? 16 : 8, rows = column_rows(to_dev(p));
+  FftLaunch c{};
+  c.tpc = threads_per_column(p, fp64 ? hold<double, true>() : hold<float, true>());
+  c.C = (int)std::max(1L, std::min(256L / c.tpc, nRows / kFftWide));
+  while (c.C > 1 && ((size_t)rows * c.C + p.N) * es > kFftLds / 2) c.C--;
+  c.T = (c.C * c.tpc + 63) / 64 * 64;
+  c.lds = ((size_t)rows * c.C + p.N) * es;
+  if (c.T > (fp64 ? 512 : 1024) || c.lds > kFftLdsMax)
+    throw Error{NPME_ERR_UNSUPPORTED, "FFT length " + std::to_string(p.N) + " does not fit a workgroup"};
+  return c;
 }
 
 // LDS of a radix-8 pass (N = 64 or 512): the columns, plus the twiddle
 // table in FP32
-static size_t pass_lds8(int N, bool fp64) { return pass_lds(N, N == 64 ? 6 : 3, fp64, false); }
-
-// L when the plan is L radix-8 stages of N = 8^L with L in {2, 3}, else 0
-static int pow8_level(const FFTPlan1D &p)
+static size_t pass_lds8(int N, bool fp64)
 {
-  if ((p.N != 64 && p.N != 512) || p.nst != (p.N == 64 ? 2 : 3)) return 0;
-  for (int i = 0; i < p.nst; i++)
-    if (p.radix[i] != 8) return 0;
-  return p.nst;
+  return (size_t)(4096) * (fp64 ? 16 : 8) + (fp64 ? 0 : (size_t)N * 8);
 }
 
-static int radix_class(const FFTPlan1D &p)
-{
-  bool r8 = true, pow2 = true;
-  for (int i = 0; i < p.nst; i++) {
-    const int r = p.radix[i];
-    if (r != 8) r8 = false;
-    if (r != 8 && r != 4 && r != 2) pow2 = false;
-  }
-  return r8 ? RC_R8 : pow2 ? RC_POW2 : RC_ALL;
-}
+// L when N = 8^L with L in {2, 3}, else 0
+static int pow8_level(const FFTPlan1D &p) { return p.N == 64 ? 2 : p.N == 512 ? 3 : 0; }
 
 static void check_int(long v, const char *what)
 {
@@ -963,7 +1276,6 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
                       const void *in, void *out, bool backward, hipStream_t s, bool pow8)
 {
   const bool rows = (g.inPos == 1 && g.outPos == 1);
-  const int lgB = lg_batch(g.N, fp64, rows);
   CGeom c;
   c.N = g.N;
   c.Lin = g.Lin;
@@ -978,19 +1290,21 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
   c.outInner = (int)g.outInner;
   c.outPos = (int)g.outPos;
   check_int(g.nCols * std::max<long>(1, g.N), "FFT pass");
-  const dim3 grid((unsigned)((g.nCols + (1 << lgB) - 1) >> lgB));
   const int L8 = pow8 ? pow8_level(plan) : 0;
+  // half the input: the pruned first stage (forward order: an even radix)
+  const bool half = !backward && 2 * g.Lin == g.N;
   if (!rows && L8 > 0 && (g.Lin == g.N || 2 * g.Lin == g.N) && g.Lout <= g.N) {
     // N = 8^L: the compile-time kernel (4096 / N columns per workgroup)
+    const dim3 grid((unsigned)((g.nCols + (4096 / g.N) - 1) / (4096 / g.N)));
     const size_t sh8 = pass_lds8(g.N, fp64);
-    const bool half = 2 * g.Lin == g.N;
+    const bool half8 = 2 * g.Lin == g.N;
 #define NPME_F8(R, LV, H)                                                                      \
   hipLaunchKernelGGL((k_fft8_cols<R, LV, H>), grid, dim3(NT), sh8, s, c,                       \
                      (const typename Cx<R>::T *)tw, (const typename Cx<R>::T *)in,            \
                      (typename Cx<R>::T *)out, (int)backward)
 #define NPME_F8L(R, LV)                                                                        \
   do {                                                                                         \
-    if (half) NPME_F8(R, LV, true);                                                            \
+    if (half8) NPME_F8(R, LV, true);                                                           \
     else NPME_F8(R, LV, false);                                                                \
   } while (0)
     if (fp64) {
@@ -1005,27 +1319,29 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
     NPME_HIP_CHECK(hipGetLastError());
     return;
   }
-  const int rc = radix_class(plan);
-  const size_t sh = pass_lds(g.N, lgB, fp64, rows);
-#define NPME_FFTC(R, ROWS, RCV)                                                                \
-  hipLaunchKernelGGL((k_fft_complex<R, ROWS, RCV>), grid, dim3(NT), sh, s, c, to_dev(plan),    \
-                     (const typename Cx<R>::T *)tw, (const typename Cx<R>::T *)in,            \
-                     (typename Cx<R>::T *)out, lgB, (int)backward)
-#define NPME_FFTC2(R, ROWS)                                                                    \
+  const PlanDev pd = to_dev(plan);
+#define NPME_FFTC(R, H)                                                                        \
   do {                                                                                         \
-    if (rc == RC_R8) NPME_FFTC(R, ROWS, RC_R8);                                                \
-    else if (rc == RC_POW2) NPME_FFTC(R, ROWS, RC_POW2);                                       \
-    else NPME_FFTC(R, ROWS, RC_ALL);                                                           \
+    if (rows)                                                                                  \
+      hipLaunchKernelGGL((k_fft_rows<R, H>), grid, dim3(l.T), l.lds, s, c, pd,                 \
+                         (const typename Cx<R>::T *)tw, (const typename Cx<R>::T *)in,        \
+                         (typename Cx<R>::T *)out, l.C, l.tpc, (int)backward);                 \
+    else                                                                                       \
+      hipLaunchKernelGGL((k_fft_cols<R, H>), grid, dim3(l.T), l.lds, s, c, pd,                 \
+                         (const typename Cx<R>::T *)tw, (const typename Cx<R>::T *)in,        \
+                         (typename Cx<R>::T *)out, l.lgB, (int)backward);                      \
   } while (0)
+  const FftLaunch l = rows ? launch_rows(plan, fp64, g.nCols) : launch_cols(plan, fp64, g.nCols);
+  const int per = rows ? l.C : 1 << l.lgB;
+  const dim3 grid((unsigned)((g.nCols + per - 1) / per));
   if (fp64) {
-    if (rows) NPME_FFTC2(double, true);
-    else NPME_FFTC2(double, false);
+    if (half) NPME_FFTC(double, true);
+    else NPME_FFTC(double, false);
   } else {
-    if (rows) NPME_FFTC2(float, true);
-    else NPME_FFTC2(float, false);
+    if (half) NPME_FFTC(float, true);
+    else NPME_FFTC(float, false);
   }
 #undef NPME_FFTC
-#undef NPME_FFTC2
   NPME_HIP_CHECK(hipGetLastError());
 }
 
@@ -1034,25 +1350,17 @@ void fft_pass_r2c_rows(bool fp64, int N, int Lin, long nRows, long inRowStride,
                        void *out, hipStream_t s)
 {
   check_int(nRows * std::max(inRowStride, outRowStride), "FFT pass");
+  if (2 * Lin != N || plan.N != N) throw Error{NPME_ERR_ARG, "R2C pass: rows of N/2 values"};
   const int nPairs = (int)(nRows / 2);
-  const int lgB = lg_batch(N, fp64, true);
-  const dim3 grid((unsigned)((nPairs + (1 << lgB) - 1) >> lgB));
-  const int rc = radix_class(plan);
-  const size_t sh = pass_lds(N, lgB, fp64, true);
-#define NPME_R2C(R, RCV)                                                                       \
-  hipLaunchKernelGGL((k_fft_r2c<R, RCV>), grid, dim3(NT), sh, s, N, Lin, nPairs, (int)inRowStride, \
+  const FftLaunch l = launch_rows(plan, fp64, nPairs);
+  const dim3 grid((unsigned)((nPairs + l.C - 1) / l.C));
+#define NPME_R2C(R)                                                                            \
+  hipLaunchKernelGGL((k_fft_r2c<R>), grid, dim3(l.T), l.lds, s, nPairs, (int)inRowStride,      \
                      (int)outRowStride, to_dev(plan), (const typename Cx<R>::T *)tw,           \
-                     (const R *)in, (typename Cx<R>::T *)out, lgB)
-#define NPME_R2C2(R)                                                                           \
-  do {                                                                                         \
-    if (rc == RC_R8) NPME_R2C(R, RC_R8);                                                       \
-    else if (rc == RC_POW2) NPME_R2C(R, RC_POW2);                                              \
-    else NPME_R2C(R, RC_ALL);                                                                  \
-  } while (0)
-  if (fp64) NPME_R2C2(double);
-  else NPME_R2C2(float);
+                     (const R *)in, (typename Cx<R>::T *)out, l.C, l.tpc)
+  if (fp64) NPME_R2C(double);
+  else NPME_R2C(float);
 #undef NPME_R2C
-#undef NPME_R2C2
   NPME_HIP_CHECK(hipGetLastError());
 }
 
@@ -1061,25 +1369,17 @@ void fft_pass_c2r_rows(bool fp64, int N, int Lout, long nRows, long inRowStride,
                        void *out, hipStream_t s)
 {
   check_int(nRows * std::max(inRowStride, outRowStride), "FFT pass");
+  if (plan.N != N) throw Error{NPME_ERR_ARG, "C2R pass: plan of another length"};
   const int nPairs = (int)(nRows / 2);
-  const int lgB = lg_batch(N, fp64, true);
-  const dim3 grid((unsigned)((nPairs + (1 << lgB) - 1) >> lgB));
-  const int rc = radix_class(plan);
-  const size_t sh = pass_lds(N, lgB, fp64, true);
-#define NPME_C2R(R, RCV)                                                                       \
-  hipLaunchKernelGGL((k_fft_c2r<R, RCV>), grid, dim3(NT), sh, s, N, Lout, nPairs, (int)inRowStride, \
+  const FftLaunch l = launch_rows(plan, fp64, nPairs);
+  const dim3 grid((unsigned)((nPairs + l.C - 1) / l.C));
+#define NPME_C2R(R)                                                                            \
+  hipLaunchKernelGGL((k_fft_c2r<R>), grid, dim3(l.T), l.lds, s, Lout, nPairs, (int)inRowStride, \
                      (int)outRowStride, to_dev(plan), (const typename Cx<R>::T *)tw,           \
-                     (const typename Cx<R>::T *)in, (R *)out, lgB)
-#define NPME_C2R2(R)                                                                           \
-  do {                                                                                         \
-    if (rc == RC_R8) NPME_C2R(R, RC_R8);                                                       \
-    else if (rc == RC_POW2) NPME_C2R(R, RC_POW2);                                              \
-    else NPME_C2R(R, RC_ALL);                                                                  \
-  } while (0)
-  if (fp64) NPME_C2R2(double);
-  else NPME_C2R2(float);
+                     (const typename Cx<R>::T *)in, (R *)out, l.C, l.tpc)
+  if (fp64) NPME_C2R(double);
+  else NPME_C2R(float);
 #undef NPME_C2R
-#undef NPME_C2R2
   NPME_HIP_CHECK(hipGetLastError());
 }
 
@@ -1098,14 +1398,12 @@ void fft_pass_convolve(bool fp64, bool complexG, int N, int Lin, long nCols, lon
   const int gm = fullG ? 2 : complexG ? 1 : 0;
   if (fullG && !complexG && (gflags & 4))
     throw Error{NPME_ERR_UNSUPPORTED, "axis-3 reversal of G needs complex data"};
-  const int lgB = lg_batch(N, fp64, false);
-  const dim3 grid((unsigned)((nCols + (1 << lgB) - 1) >> lgB));
-  const int rc = radix_class(plan);
-  const size_t sh = pass_lds(N, lgB, fp64, false);
+  if (2 * Lin != N || plan.N != N) throw Error{NPME_ERR_ARG, "convolution pass: columns of N/2 values"};
   // the axis-3 length of complex data (0 for the R2C data of real kernels)
   const int N3fold = complexG ? (int)Kv : 0;
   const int L8 = pow8 ? pow8_level(plan) : 0;
-  if (L8 > 0 && 2 * Lin == N) {
+  if (L8 > 0) {
+    const dim3 grid((unsigned)((nCols + (4096 / N) - 1) / (4096 / N)));
     const size_t sh8 = pass_lds8(N, fp64);
 #define NPME_C8(R, LV, GMV)                                                                    \
   hipLaunchKernelGGL((k_fft8_conv<R, LV, GMV>), grid, dim3(NT), sh8, s, (int)nCols,           \
@@ -1130,53 +1428,48 @@ void fft_pass_convolve(bool fp64, bool complexG, int N, int Lin, long nCols, lon
     NPME_HIP_CHECK(hipGetLastError());
     return;
   }
-#define NPME_CONV(R, GMV, RCV)                                                                 \
-  hipLaunchKernelGGL((k_fft_conv<R, GMV, RCV>), grid, dim3(NT), sh, s, N, Lin, (int)nCols,     \
+  const FftLaunch l = launch_cols(plan, fp64, nCols);
+  const dim3 grid((unsigned)((nCols + (1 << l.lgB) - 1) >> l.lgB));
+#define NPME_CONV(R, GMV)                                                                      \
+  hipLaunchKernelGGL((k_fft_conv<R, GMV>), grid, dim3(l.T), l.lds, s, (int)nCols,              \
                      (int)pos_stride, N2, gflags, (int)C3, (int)Kv, N3fold, to_dev(plan),       \
-                     (const typename Cx<R>::T *)tw, G, (typename Cx<R>::T *)data, lgB)
-#define NPME_CONV2(R, GMV)                                                                     \
-  do {                                                                                         \
-    if (rc == RC_R8) NPME_CONV(R, GMV, RC_R8);                                                 \
-    else if (rc == RC_POW2) NPME_CONV(R, GMV, RC_POW2);                                        \
-    else NPME_CONV(R, GMV, RC_ALL);                                                            \
-  } while (0)
+                     (const typename Cx<R>::T *)tw, G, (typename Cx<R>::T *)data, l.lgB)
 #define NPME_CONVG(R)                                                                          \
   do {                                                                                         \
-    if (gm == 2) NPME_CONV2(R, 2);                                                             \
-    else if (gm == 1) NPME_CONV2(R, 1);                                                        \
-    else NPME_CONV2(R, 0);                                                                     \
+    if (gm == 2) NPME_CONV(R, 2);                                                              \
+    else if (gm == 1) NPME_CONV(R, 1);                                                         \
+    else NPME_CONV(R, 0);                                                                      \
   } while (0)
   if (fp64) NPME_CONVG(double);
   else NPME_CONVG(float);
 #undef NPME_CONVG
 #undef NPME_CONV
-#undef NPME_CONV2
+  NPME_HIP_CHECK(hipGetLastError());
+}
+
+template <bool PAIR>
+static void pass_even(int N, long nCols, long nInner, long outer, long inner, long pos,
+                      const FFTPlan1D &plan, const void *tw, void *data, hipStream_t s)
+{
+  check_int(nCols * (long)(N / 2 + 1), "FFT pass");
+  const long cols = PAIR ? (nCols + 1) / 2 : nCols;
+  const FftLaunch l = launch_cols(plan, true, cols);
+  const dim3 grid((unsigned)((cols + (1 << l.lgB) - 1) >> l.lgB));
+  hipLaunchKernelGGL(k_fft_even<PAIR>, grid, dim3(l.T), l.lds, s, (int)nCols, (int)nInner, (int)outer,
+                     (int)inner, (int)pos, to_dev(plan), (const double2 *)tw, data, l.lgB);
   NPME_HIP_CHECK(hipGetLastError());
 }
 
 void fft_pass_even_real(int N, long nCols, long nInner, long outer, long inner, long pos,
                         const FFTPlan1D &plan, const void *tw, double *data, hipStream_t s)
 {
-  check_int(nCols * (long)(N / 2 + 1), "FFT pass");
-  const int lgB = lg_batch(N, true, false);
-  const long pairs = (nCols + 1) / 2;
-  const dim3 grid((unsigned)((pairs + (1 << lgB) - 1) >> lgB));
-  const size_t sh = lds_bytes(N, lgB, true, false);
-  hipLaunchKernelGGL(k_fft_even_pair, grid, dim3(NT), sh, s, N, (int)nCols, (int)nInner, (int)outer,
-                     (int)inner, (int)pos, to_dev(plan), (const double2 *)tw, data, lgB);
-  NPME_HIP_CHECK(hipGetLastError());
+  pass_even<true>(N, nCols, nInner, outer, inner, pos, plan, tw, data, s);
 }
 
 void fft_pass_even(int N, long nCols, long nInner, long outer, long inner, long pos,
                    const FFTPlan1D &plan, const void *tw, void *data, hipStream_t s)
 {
-  check_int(nCols * (long)(N / 2 + 1), "FFT pass");
-  const int lgB = lg_batch(N, true, false);
-  const dim3 grid((unsigned)((nCols + (1 << lgB) - 1) >> lgB));
-  const size_t sh = lds_bytes(N, lgB, true, false);
-  hipLaunchKernelGGL(k_fft_even, grid, dim3(NT), sh, s, N, (int)nCols, (int)nInner, (int)outer,
-                     (int)inner, (int)pos, to_dev(plan), (const double2 *)tw, (double2 *)data, lgB);
-  NPME_HIP_CHECK(hipGetLastError());
+  pass_even<false>(N, nCols, nInner, outer, inner, pos, plan, tw, data, s);
 }
 
 }  // namespace npme
