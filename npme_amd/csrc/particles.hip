@@ -19,6 +19,11 @@
 
 namespace npme {
 
+// pair-function variants of the device kernels (besides the kernel kinds):
+// Helmholtz with a real wave number, and r^alpha with 2 alpha a small integer
+enum { KIND_HELMHOLTZ_REAL = 32, KIND_RALPHA_HALF = 33 };
+constexpr bool pair_is_complex(int kind) { return kind == KIND_HELMHOLTZ_REAL || kind_is_complex(kind); }
+
 template <typename R> struct V4t;
 template <> struct V4t<float> { using T = float4; };
 template <> struct V4t<double> { using T = double4; };
@@ -39,6 +44,8 @@ struct DirectDev {
   double fxInvD;     // fxInv in FP64 (scale of the list walk's gradient sums)
   float fxClose2u;   // list walk: squared distance in fixed-point units below which
                      // a pair adds the residuals (2^48: pairs closer than 2^24 units)
+  float k0q[2];      // k0r 2 / pi split in two FP32 parts (phase in quarter turns)
+  int raPow, raHalf; // KIND_RALPHA_HALF: alpha = raPow + raHalf / 2
   const void *utab;  // user kernels: short-range table in the working precision
   int utS;           // pieces per octave of the table
   double invRdir;
@@ -164,8 +171,6 @@ void launch_gather_q(bool fp64, bool complexK, size_t n, const int *perm, const 
 
 // ------------------------------------------------------------------ direct
 template <typename Real> __device__ __forceinline__ Real rsqrt_r(Real x);
-__device__ __forceinline__ void sincos_r(float x, float *s, float *c) { sincosf(x, s, c); }
-__device__ __forceinline__ void sincos_r(double x, double *s, double *c) { sincos(x, s, c); }
 // v_rsq_f32 (1 ulp): r2 of a pair is never denormal, so the range fix-up
 // of rsqrtf is not needed
 template <> __device__ __forceinline__ float rsqrt_r<float>(float x) { return __builtin_amdgcn_rsqf(x); }
@@ -242,7 +247,7 @@ __global__ __launch_bounds__(256) void k_direct(DirectDev p, size_t n,
                                                 int nP, double csA, double *__restrict__ Vdir)
 {
   using V4 = typename V4t<Real>::T;
-  constexpr bool CX = kind_is_complex(KIND);
+  constexpr bool CX = pair_is_complex(KIND);
   const int lane = threadIdx.x & 63;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   const int blk = wg * 4 + (threadIdx.x >> 6);
@@ -372,7 +377,23 @@ static DirectDev direct_dev(const DirectParams &p)
   d.eshift = p.nlEshift;
   d.fxInvD = p.fxInv;
   d.fxClose2u = 281474976710656.0f;  // 2^48
+  const double kq = p.k0r * 0.63661977236758134308;
+  d.k0q[0] = (float)kq;
+  d.k0q[1] = (float)(kq - (double)d.k0q[0]);
+  d.raPow = (int)std::floor(p.alpha);
+  d.raHalf = 2.0 * p.alpha != 2.0 * d.raPow;
   return d;
+}
+
+// the FP32 pair function of a kernel: KIND_HELMHOLTZ without damping skips
+// the exponential; r^alpha with 2 alpha an integer, |alpha| <= 3 (a product of
+// at most three rounded factors) needs no pow
+static int pair_kind32(const DirectParams &p)
+{
+  if (p.kind == KIND_HELMHOLTZ && p.k0i == 0.0) return KIND_HELMHOLTZ_REAL;
+  if (p.kind == KIND_RALPHA && std::fabs(p.alpha) <= 3.0 && 2.0 * p.alpha == std::floor(2.0 * p.alpha))
+    return KIND_RALPHA_HALF;
+  return p.kind;
 }
 
 void launch_direct(bool fp64, const DirectParams &p, size_t n, const void *src, const void *res,
@@ -402,7 +423,10 @@ void launch_direct(bool fp64, const DirectParams &p, size_t n, const void *src, 
     else if (p.kind == KIND_USER_CX) NPME_DIRECT_D(double, KIND_USER_CX, false, 4);
     else NPME_DIRECT(double, KIND_HELMHOLTZ, false);
   } else {
+    const int kind = pair_kind32(p);
     if (p.kind == KIND_LAPLACE) NPME_DIRECT(float, KIND_LAPLACE, true);
+    else if (kind == KIND_RALPHA_HALF) NPME_DIRECT(float, KIND_RALPHA_HALF, true);
+    else if (kind == KIND_HELMHOLTZ_REAL) NPME_DIRECT(float, KIND_HELMHOLTZ_REAL, true);
     else if (p.kind == KIND_LAPLACE_ERF) NPME_DIRECT_D(float, KIND_LAPLACE_ERF, true, 8);
     else if (p.kind == KIND_RALPHA) NPME_DIRECT(float, KIND_RALPHA, true);
     else if (p.kind == KIND_USER) NPME_DIRECT_D(float, KIND_USER, true, 4);
@@ -980,6 +1004,66 @@ __device__ __forceinline__ void user_sr(const DirectDev &p, Real r2, Real *f)
   if (!CXU) f[1] = f[3] = (Real)0;
 }
 
+// 1/r and r of r2 in FP32, each within about half an ulp: the hardware
+// estimate (1 ulp) and one correction step
+__device__ __forceinline__ void inv_and_root(float r2, float &ri, float &r)
+{
+  ri = __builtin_amdgcn_rsqf(r2);
+  r = r2 * ri;
+  r = fmaf(0.5f * ri, fmaf(-r, r, r2), r);
+  ri = fmaf(ri, fmaf(-r, ri, 1.0f), ri);
+}
+
+// a number as the sum of two FP32 numbers (lo below half an ulp of hi, or a
+// little more): products keep about twice FP32's precision, so a chain of
+// them is rounded once at its end
+struct Two {
+  float hi, lo;
+};
+__device__ __forceinline__ Two two_mul(Two a, Two b)
+{
+  const float p = a.hi * b.hi;
+  return {p, fmaf(a.hi, b.hi, -p) + fmaf(a.hi, b.lo, a.lo * b.hi)};
+}
+// square root of x (its low part from the residual), and 1 / sqrt(x)
+__device__ __forceinline__ void two_root(Two x, Two &rt, Two &inv)
+{
+  const float y = __builtin_amdgcn_rsqf(x.hi);
+  rt.hi = x.hi * y;
+  rt.lo = (fmaf(-rt.hi, rt.hi, x.hi) + x.lo) * (0.5f * y);
+  inv.hi = y;
+  inv.lo = y * fmaf(-rt.lo, y, fmaf(-rt.hi, y, 1.0f));
+}
+
+// cos and sin of pi/2 (khi + klo) r in FP32.  The phase in quarter turns is
+// r khi exactly as a sum of two FP32 numbers (fma), so removing the nearest
+// integer leaves the fraction t in [-1/2, 1/2] with an error of half an ulp
+// of 1/2 whatever the phase, as good as a reduction in FP64; sin and cos of
+// pi/2 t are minimax polynomials in t^2 (relative errors 3.8e-9 and 6.4e-11,
+// fitted by Lawson's iteration; FP32 evaluation 4.2e-8 and 5.7e-8 absolute).
+// ~25 instructions, against ~95 for the FP64 reduction and the library's
+// sincosf with its own.
+__device__ __forceinline__ void phase_sincos(float r, float khi, float klo, float &sn, float &cn)
+{
+#pragma clang fp contract(off)
+  const float pq = r * khi;
+  const float n = __builtin_rintf(pq);
+  const float t = (pq - n) + fmaf(r, klo, fmaf(r, khi, -pq));
+  const float s = t * t;
+  float a = fmaf(s, -0.0046048265110679235f, 0.07968141056178463f);
+  a = fmaf(s, a, -0.6459636300573146f);
+  a = fmaf(s, a, -4.371139e-08f);  // pi/2 - (float)(pi/2)
+  a = fmaf(t, 1.5707963267948966f, t * a);
+  float b = fmaf(s, 0.0009037649755624962f, -0.020860164437089795f);
+  b = fmaf(s, b, 0.25366922587909174f);
+  b = fmaf(s, b, -1.2337005425945717f);
+  b = fmaf(s, b, 1.0f);
+  const unsigned q = (unsigned)(int)n;
+  const float x = (q & 1u) ? a : b, y = (q & 1u) ? b : a;
+  cn = __uint_as_float(__float_as_uint(x) ^ (((q + 1u) & 2u) << 30));
+  sn = __uint_as_float(__float_as_uint(y) ^ ((q & 2u) << 30));
+}
+
 // short-range DM pair term of one source (charge qr + i qim) at offset
 // (rx, ry, rz), r2 = |r|^2 < Rdir^2, added to part: V and grad (real), or
 // (re, im) of V, d/dx, d/dy, d/dz (complex)
@@ -1036,6 +1120,26 @@ __device__ __forceinline__ void pair_sr(const DirectDev &p, Real rx, Real ry, Re
     part[5] += ry * gi;
     part[6] += rz * gr;
     part[7] += rz * gi;
+  } else if constexpr (KIND == KIND_RALPHA_HALF) {
+    // FP32: r^alpha = r^raPow sqrt(r)^raHalf by hardware roots and products
+    // in two-part arithmetic, rounded once (the branches are uniform).  r^0.5
+    // at 200k charges: 121 -> 49 us against pow and a division
+    Two r, ri, fe = {1.0f, 0.0f};
+    two_root({r2, 0.0f}, r, ri);
+    if (p.raHalf) {
+      Two hi;
+      two_root(r, fe, hi);
+    }
+    const Two m = p.raPow >= 0 ? r : ri;
+    for (int k = abs(p.raPow); k > 0; k--) fe = two_mul(fe, m);
+    const Two fd = two_mul(fe, two_mul(ri, ri));
+    const Real f0 = (fe.hi - horner_top<Real, MAXD>(topA, coef_a<Real>(p), r2)) + fe.lo;
+    const Real f1 = (Real)p.alpha * (fd.hi + fd.lo) - horner_top<Real, MAXD>(topB, coef_b<Real>(p), r2);
+    const Real fq = f1 * qr;
+    part[0] += f0 * qr;
+    part[1] += rx * fq;
+    part[2] += ry * fq;
+    part[3] += rz * fq;
   } else if constexpr (KIND == KIND_RALPHA) {
     const Real fe = pow(r2, (Real)(0.5 * p.alpha));
     const Real f0 = fe - horner_top<Real, MAXD>(topA, coef_a<Real>(p), r2);
@@ -1048,17 +1152,22 @@ __device__ __forceinline__ void pair_sr(const DirectDev &p, Real rx, Real ry, Re
   } else {
     (void)topA;
     (void)topB;
-    // exp(i k0 r)/r with the phase k0r r reduced modulo 2 pi in FP64
-    const Real r = sqrt(r2);
-    const Real ri = (Real)1 / r;
-    const double ph = p.k0r * (double)r;
-    const double red = ph - 6.283185307179586477 * rint(ph * 0.15915494309189533577);
-    Real sn, cn;
-    sincos_r((Real)red, &sn, &cn);
-    const Real damp = exp((Real)(-p.k0i) * r) * ri;
+    // exp(i k0 r)/r; FP64: the phase k0r r reduced modulo 2 pi first
+    Real r, ri, sn, cn;
+    if constexpr (sizeof(Real) == 4) {
+      inv_and_root(r2, ri, r);
+      phase_sincos(r, p.k0q[0], p.k0q[1], sn, cn);
+    } else {
+      r = sqrt(r2);
+      ri = (Real)1 / r;
+      const double ph = p.k0r * (double)r;
+      const double red = ph - 6.283185307179586477 * rint(ph * 0.15915494309189533577);
+      sincos(red, &sn, &cn);
+    }
+    const Real damp = KIND == KIND_HELMHOLTZ_REAL ? ri : exp((Real)(-p.k0i) * r) * ri;
     const Real fr = damp * cn, fi = damp * sn;
     const Real k0r = (Real)p.k0r, k0i = (Real)p.k0i;
-    const Real ikr = -k0i - ri, iki = k0r;  // i k0 - 1/r
+    const Real ikr = KIND == KIND_HELMHOLTZ_REAL ? -ri : -k0i - ri, iki = k0r;  // i k0 - 1/r
     const Real f1r = (ikr * fr - iki * fi) * ri, f1i = (ikr * fi + iki * fr) * ri;
     Real pr, pim, br, bi;
     horner_fix_cx<Real, MAXD>(coef_a<Real>(p), r2, pr, pim);
@@ -1092,7 +1201,7 @@ __device__ __forceinline__ void direct_slice(const DirectDev &p, size_t n, size_
                                              Real topB)
 {
   using V4 = typename V4t<Real>::T;
-  constexpr bool CX = kind_is_complex(KIND);
+  constexpr bool CX = pair_is_complex(KIND);
   const size_t s = slice * kNlSlice + (lane >> kNlTeamLog);
   const bool tvalid = s < n;
   const size_t tt = tvalid ? s : slice * kNlSlice;
@@ -1254,8 +1363,13 @@ __device__ __forceinline__ void direct_slice(const DirectDev &p, size_t n, size_
 // grid of a wavefront per slice used here.  (Grids of a few workgroups per
 // CU, which leave wave slots to the reciprocal sum's kernels on the other
 // stream, measured slower at N = 1M.)
+// FP32 Helmholtz is held to 128 VGPRs (the compiler's own choice is 129 to
+// 132, 3 wavefronts per SIMD: 1.52 against 1.42 ms at 500k charges, 5.6e8
+// pairs, where pair arithmetic, ~100 instructions each, is the bound; the
+// library's sincosf, exp, division and FP64 reduction had taken 2.22 ms).
 template <typename Real, int KIND, bool FIXP, int MAXD>
-__global__ __launch_bounds__(256) void k_direct_nl(DirectDev p, size_t n,
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(pair_is_complex(KIND) && sizeof(Real) == 4 ? 4 : 1))) void k_direct_nl(DirectDev p, size_t n,
                                                    const typename V4t<Real>::T *__restrict__ src,
                                                    const float4 *__restrict__ res,
                                                    const Real *__restrict__ qi,
@@ -1311,7 +1425,10 @@ void launch_direct_nl(bool fp64, const DirectParams &p, size_t n, const void *sr
     else if (p.kind == KIND_USER_CX) NPME_DNL_D(double, KIND_USER_CX, false, 4);
     else NPME_DNL(double, KIND_HELMHOLTZ, false);
   } else {
+    const int kind = pair_kind32(p);
     if (p.kind == KIND_LAPLACE) NPME_DNL(float, KIND_LAPLACE, true);
+    else if (kind == KIND_RALPHA_HALF) NPME_DNL(float, KIND_RALPHA_HALF, true);
+    else if (kind == KIND_HELMHOLTZ_REAL) NPME_DNL(float, KIND_HELMHOLTZ_REAL, true);
     else if (p.kind == KIND_LAPLACE_ERF) NPME_DNL_D(float, KIND_LAPLACE_ERF, true, 4);
     else if (p.kind == KIND_RALPHA) NPME_DNL(float, KIND_RALPHA, true);
     else if (p.kind == KIND_USER) NPME_DNL_D(float, KIND_USER, true, 4);
@@ -1436,7 +1553,7 @@ __global__ __launch_bounds__(256) void k_direct_refpairs(DirectDev p, size_t n, 
   const int4 c = cell[s];
   const long cl = ((long)c.x * p.nb1 + c.y) * p.nb2 + c.z;
   const double4 me = xs[s];
-  constexpr bool CX = kind_is_complex(KIND);
+  constexpr bool CX = pair_is_complex(KIND);
   double part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   for (int o = 0; o < nOff; o++) {
     if (!((flags[cl * W + (o >> 5)] >> (o & 31)) & 1u)) continue;
@@ -2254,7 +2371,7 @@ __global__ __launch_bounds__(256) void k_exact(double alpha, double k0r, double 
                                                const long *__restrict__ idx,
                                                double *__restrict__ Vout)
 {
-  constexpr bool CX = kind_is_complex(KIND);
+  constexpr bool CX = pair_is_complex(KIND);
   __shared__ double sx[256], sy[256], sz[256], sq[256], sqi[256];
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool active = t < nt;

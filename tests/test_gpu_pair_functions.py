@@ -1,0 +1,52 @@
+"""The FP32 pair functions that replace library calls (mixed precision):
+r^alpha with 2 alpha an integer (roots and products), the ones beside them
+that still call pow, and Helmholtz with and without damping, phases up to a turn, in the neighbour-list walk and the cell rows, against the
+oracle on the same grid.
+
+Bound: each FP32 pair term is within a few 6e-8 of its value; the sums of a
+few hundred terms of either sign stay within 1e-6 of V and 1e-5 of the
+gradient, the bounds of the mixed form elsewhere.  (Kernels that grow faster
+than r^1.5 are left out: there the smooth part dwarfs the pair terms, and the
+FP32 grid alone, 1.2e-6 for r^3, decides the error; and so are wave numbers
+beyond a turn inside the cutoff, where the matched polynomials cancel.)"""
+import numpy as np
+import pytest
+
+from conftest import uniform_box
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(oracle, kind, ko, coord, q, **kw):
+    import npme_amd as N
+    cx = kind == "Helmholtz"
+    k = N.NPME_KeywordInput(calcType="pme", funcType=kind, EwaldSplit="DerivMatch", Rdir=6.0, BnOrder=6,
+                            tol=1e-6, precision="mixed", N1=64, N2=64, N3=64, n1=16, n2=16, n3=16,
+                            nDeriv=6, **kw)
+    charge = {"chargeComplex": q} if cx else {"chargeReal": q}
+    assert N.NPME_AddMissingKeywords(k, len(q), coord, **charge), N.npme_last_error()
+    h = (N.NPME_Interface_SetUpComplexKernel if cx else N.NPME_Interface_SetUpRealKernel)(k, len(q), coord)
+    assert h is not None, N.npme_last_error()
+    m = oracle.compare_v(oracle.calcv(ko, (64, 64, 64), 6, coord, q), h.calcv(q))
+    print(m["relV"], m["reldV"])
+    assert m["relV"] < 1e-6 and m["reldV"] < 1e-5, m
+
+
+@pytest.mark.parametrize("lists", ["on", "off"])
+@pytest.mark.parametrize("alpha", [0.5, 1.5, -0.5, -2.5, 1.0, -2.0, -3.0, 0.3, -3.5])
+def test_ralpha_pairs(oracle, alpha, lists):
+    print("case ralpha pairs", alpha, lists, flush=True)
+    coord, q = uniform_box(1500, 20.0)
+    _run(oracle, "Ralpha", oracle.kernel(oracle.RALPHA, 6, 6.0, alpha=alpha), coord, q, alpha=alpha,
+         neighborList=lists)
+
+
+@pytest.mark.parametrize("lists", ["on", "off"])
+@pytest.mark.parametrize("k0", [0.01, 0.5, 1.0, 1.1 + 0.2j, 0.3 + 0.01j])
+def test_helmholtz_pairs(oracle, k0, lists):
+    print("case helmholtz pairs", k0, lists, flush=True)
+    coord, q = uniform_box(1500, 20.0)
+    q = q + 1j * uniform_box(1500, 20.0, 7, 8)[1]
+    k0 = complex(k0)
+    _run(oracle, "Helmholtz", oracle.kernel(oracle.HELMHOLTZ, 6, 6.0, k0=k0), coord, q, k0_r=k0.real,
+         k0_i=k0.imag, neighborList=lists)
