@@ -319,6 +319,7 @@ struct Handle {
   void *d_frac = nullptr;        // [n] float4/double4 fractional spline arguments
   int *d_tileStart = nullptr;    // [ntiles + 1]
   int *d_tileList = nullptr;     // [nlist]
+  size_t nTileEntries = 0;       // its length
   int TI = 16;                   // interpolation tile edge
   int nti[3] = {0, 0, 0};
   int *d_itileStart = nullptr;   // [ntiles + 1] charges per interpolation tile
@@ -574,7 +575,7 @@ void launch_direct_nl(bool fp64, const DirectParams &p, size_t n, const void *sr
 void launch_count_pairs(const DirectParams &p, size_t n, const int4 *cell, const int *cellStart,
                         const double4 *xs, unsigned long long *total, hipStream_t s);
 void launch_spread(bool fp64, bool complexK, long Bn, const long M[3], const int T[3],
-                   const int nt[3], const int *tileStart, const int *tileList, const void *qre,
+                   const int nt[3], const int *tileStart, const int *tileList, size_t entries, const void *qre,
                    const void *qim, const int4 *ms, const void *frac, void *grid, hipStream_t s);
 void launch_interp(bool fp64, bool complexK, long Bn, const long M[3], const double C[3], int T,
                    const int nt[3], const int *tileStart, const int *tileList, const int4 *ms,

@@ -1778,8 +1778,31 @@ __device__ __forceinline__ void bsp_weights_grad(int n, double t, Real *B, Real 
 // q w1[i] w2[j] w3[k] into its column.
 constexpr int TS = 8;
 
-template <typename Real, bool CX, int BN>
-__global__ __launch_bounds__(64) void k_spread(int BnRun, long M1, long M2, long M3, int nt1, int nt2,
+// W wavefronts share a tile: wavefront w takes the chunks w, w + W, ... of
+// its list, each with staging rows of its own, and the wavefronts' FP64 sums
+// are added in order at the end (spread_waves: sets whose tiles are too few
+// to fill the chip).  A wavefront's LDS accesses execute in program order, so
+// rows written by some of its lanes and read by others need no barrier, only
+// that the compiler keeps the order.
+__device__ __forceinline__ void wave_lds_order()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the W wavefronts' sums of element e of lane l, added in order: red holds
+// [wavefront][E][64] doubles
+template <int W, int E> __device__ __forceinline__ double spread_sum(const double *red, int e, int l)
+{
+  double v = red[e * 64 + l];
+#pragma unroll
+  for (int w = 1; w < W; w++) v += red[(w * E + e) * 64 + l];
+  return v;
+}
+
+template <typename Real, bool CX, int BN, int W>
+__global__ __launch_bounds__(64 * W) void k_spread(int BnRun, long M1, long M2, long M3, int nt1, int nt2,
                                                int nt3, const int *__restrict__ tileStart,
                                                const int *__restrict__ tileList,
                                                const Real *__restrict__ qre,
@@ -1789,22 +1812,27 @@ __global__ __launch_bounds__(64) void k_spread(int BnRun, long M1, long M2, long
                                                Real *__restrict__ grid)
 {
   // per staged charge: w1[8], w2[8], w3[8] restricted to the tile, q, q_im
-  __shared__ __align__(16) Real w[64][3 * TS];
-  __shared__ Real qs[64][2];
+  constexpr int E = CX ? 2 * TS : TS;
+  constexpr size_t rowB = 64 * 3 * TS * sizeof(Real), waveB = rowB + 64 * 2 * sizeof(Real);
+  constexpr size_t redB = W > 1 ? (size_t)W * E * 64 * sizeof(double) : 0;
+  __shared__ __align__(16) char mem[W * waveB > redB ? W * waveB : redB];
+  const int wv = W > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0, l = threadIdx.x & 63;
+  Real(*w)[3 * TS] = reinterpret_cast<Real(*)[3 * TS]>(mem + wv * waveB);
+  Real(*qs)[2] = reinterpret_cast<Real(*)[2]>(mem + wv * waveB + rowB);
   const int Bn = BN > 0 ? BN : BnRun;
   constexpr int BA = BN > 0 ? BN : 16;
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   const int t3 = t % nt3, t2 = (t / nt3) % nt2, t1 = t / (nt3 * nt2);
   const int u1 = t1 * TS, u2 = t2 * TS, u3 = t3 * TS;
-  const int li = threadIdx.x / TS, lj = threadIdx.x % TS;
+  const int li = l / TS, lj = l % TS;
   double acc[2 * TS];
 #pragma unroll
   for (int k = 0; k < 2 * TS; k++) acc[k] = 0;
   const int beg = tileStart[t], end = tileStart[t + 1];
-  for (int base = beg; base < end; base += 64) {
+  for (int base = beg + 64 * wv; base < end; base += 64 * W) {
     const int cnt = min(64, end - base);
-    if ((int)threadIdx.x < cnt) {
-      const int s = tileList[base + threadIdx.x];
+    if (l < cnt) {
+      const int s = tileList[base + l];
       const int4 m0 = ms[s];
       const typename V4t<Real>::T f = frac[s];
       Real sh[BA];
@@ -1822,13 +1850,13 @@ __global__ __launch_bounds__(64) void k_spread(int BnRun, long M1, long M2, long
 #pragma unroll
           for (int j = 0; j < BA; j++)
             if (j == idx && j < Bn) v = sh[j];
-          w[threadIdx.x][d * TS + k] = v;
+          w[l][d * TS + k] = v;
         }
       }
-      qs[threadIdx.x][0] = qre[s];
-      qs[threadIdx.x][1] = CX ? qim[s] : (Real)0;
+      qs[l][0] = qre[s];
+      qs[l][1] = CX ? qim[s] : (Real)0;
     }
-    __syncthreads();
+    wave_lds_order();
     // FP32 (or FP64) sums over the chunk, carried into FP64 per chunk
     Real part[2 * TS];
 #pragma unroll
@@ -1853,25 +1881,29 @@ __global__ __launch_bounds__(64) void k_spread(int BnRun, long M1, long M2, long
     }
 #pragma unroll
     for (int k = 0; k < (CX ? 2 * TS : TS); k++) acc[k] += (double)part[k];
-    __syncthreads();
+    wave_lds_order();
   }
   const long p1 = u1 + li, p2 = u2 + lj;
-  if (p1 < M1 && p2 < M2) {
-    const long row = (p1 * M2 + p2) * M3;
+  const long row = (p1 * M2 + p2) * M3;
+  const bool in = p1 < M1 && p2 < M2;
+  constexpr int P = CX ? 2 : 1;
+  if constexpr (W == 1) {
 #pragma unroll
-    for (int k = 0; k < TS; k++) {
-      const long p3 = u3 + k;
-      if (p3 < M3) {
-        if (CX) {
-          grid[2 * (row + p3)] = (Real)acc[2 * k];
-          grid[2 * (row + p3) + 1] = (Real)acc[2 * k + 1];
-        } else {
-          grid[row + p3] = (Real)acc[k];
-        }
-      }
+    for (int e = 0; e < E; e++)
+      if (in && u3 + e / P < M3) grid[P * (row + u3) + e] = (Real)acc[e];
+  } else {
+    double *red = reinterpret_cast<double *>(mem);
+    __syncthreads();  // every wavefront is done with its rows
+#pragma unroll
+    for (int e = 0; e < E; e++) red[(wv * E + e) * 64 + l] = acc[e];
+    __syncthreads();
+    for (int e = wv; e < E; e += W) {
+      const double v = spread_sum<W, E>(red, e, l);
+      if (in && u3 + e / P < M3) grid[P * (row + u3) + e] = (Real)v;
     }
   }
 }
+
 
 // Matrix-core spreading (FP32, real charges).  A tile of 16 x 8 x 8 grid
 // points is one wavefront; over the charges c listed for the tile
@@ -1885,8 +1917,8 @@ __global__ __launch_bounds__(64) void k_spread(int BnRun, long M1, long M2, long
 // row per charge, zero outside the spline window), then runs the products;
 // the FP32 block sums are carried into FP64 per chunk.
 typedef float npme_f4 __attribute__((ext_vector_type(4)));
-template <int BN>
-__global__ __launch_bounds__(64) void k_spread_mfma(int BnRun, long M1, long M2, long M3, int nt1,
+template <int BN, int W>
+__global__ __launch_bounds__(64 * W) void k_spread_mfma(int BnRun, long M1, long M2, long M3, int nt1,
                                                     int nt2, int nt3,
                                                     const int *__restrict__ tileStart,
                                                     const int *__restrict__ tileList,
@@ -1900,7 +1932,10 @@ __global__ __launch_bounds__(64) void k_spread_mfma(int BnRun, long M1, long M2,
   // four groups of a step read four consecutive rows (no bank conflicts).
   // The three row blocks are one 8 KB block, cleared per chunk by the
   // wavefront in contiguous 1 KB runs
-  __shared__ __align__(16) float stage[64 * (TX + TY + TZ)];
+  constexpr int ROW = 64 * (TX + TY + TZ);
+  __shared__ __align__(16) float stages[W * ROW];
+  const int wv = W > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+  float *stage = stages + wv * ROW;
   float(*sA)[TX] = reinterpret_cast<float(*)[TX]>(stage);
   float(*sW2)[TY] = reinterpret_cast<float(*)[TY]>(stage + 64 * TX);
   float(*sW3)[TZ] = reinterpret_cast<float(*)[TZ]>(stage + 64 * (TX + TY));
@@ -1909,7 +1944,7 @@ __global__ __launch_bounds__(64) void k_spread_mfma(int BnRun, long M1, long M2,
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   const int t3 = t % nt3, t2 = (t / nt3) % nt2, t1 = t / (nt3 * nt2);
   const int u1 = t1 * TX, u2 = t2 * TY, u3 = t3 * TZ;
-  const int l = threadIdx.x, n16 = l & 15, kq = l >> 4;
+  const int l = threadIdx.x & 63, n16 = l & 15, kq = l >> 4;
   double acc[4][4];
 #pragma unroll
   for (int b = 0; b < 4; b++)
@@ -1929,16 +1964,14 @@ __global__ __launch_bounds__(64) void k_spread_mfma(int BnRun, long M1, long M2,
       q = qre[c];
     }
   };
-  fetch(beg, cm, cf, cq);
-  for (int base = beg; base < end; base += 64) {
+  fetch(beg + 64 * wv, cm, cf, cq);
+  for (int base = beg + 64 * wv; base < end; base += 64 * W) {
     const int cnt = min(64, end - base);
     // row l: zeros, then the spline window of charge l at its tile slots.
     // The w2 row is stored as (w2[0], w2[2], w2[4], w2[6], w2[1], w2[3],
     // w2[5], w2[7]): a lane's four B columns j = 2b + h (h = n16 / 8) are
     // then one 16-byte read
     {
-      // the workgroup is this one wavefront, whose LDS accesses execute in
-      // program order, so the window writes below follow the clearing
       const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int k = 0; k < (TX + TY + TZ) / 4; k++) reinterpret_cast<float4 *>(stage)[64 * k + l] = z4;
@@ -1966,8 +1999,8 @@ __global__ __launch_bounds__(64) void k_spread_mfma(int BnRun, long M1, long M2,
       for (int j = 0; j < BA; j++)
         if (j < Bn && off + j >= 0 && off + j < TZ) sW3[l][off + j] = sh[j];
     }
-    __syncthreads();
-    fetch(base + 64, cm, cf, cq);
+    wave_lds_order();
+    fetch(base + 64 * W, cm, cf, cq);
     npme_f4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = d0, d2 = d0, d3 = d0;
     const int nstep = (cnt + 3) >> 2;  // rows past cnt are zero
 #pragma unroll 2
@@ -1986,17 +2019,26 @@ __global__ __launch_bounds__(64) void k_spread_mfma(int BnRun, long M1, long M2,
     for (int b = 0; b < 4; b++)
 #pragma unroll
       for (int r = 0; r < 4; r++) acc[b][r] += (double)dd[b][r];
-    __syncthreads();  // the rows are rewritten by the next chunk
+    wave_lds_order();  // the rows are rewritten by the next chunk
   }
   const long p3 = u3 + (n16 & 7);
+  auto put = [&](int b, int r, double v) {
+    const long p2 = u2 + 2 * b + (n16 >> 3), p1 = u1 + 4 * kq + r;
+    if (p1 < M1 && p2 < M2 && p3 < M3) grid[(p1 * M2 + p2) * M3 + p3] = (float)v;
+  };
+  if constexpr (W == 1) {
 #pragma unroll
-  for (int b = 0; b < 4; b++) {
-    const long p2 = u2 + 2 * b + (n16 >> 3);
+    for (int b = 0; b < 4; b++)
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const long p1 = u1 + 4 * kq + r;
-      if (p1 < M1 && p2 < M2 && p3 < M3) grid[(p1 * M2 + p2) * M3 + p3] = (float)acc[b][r];
-    }
+      for (int r = 0; r < 4; r++) put(b, r, acc[b][r]);
+  } else {
+    static_assert(ROW * sizeof(float) >= 16 * 64 * sizeof(double), "sums fit the staging rows");
+    double *red = reinterpret_cast<double *>(stages);
+    __syncthreads();  // every wavefront is done with its rows
+#pragma unroll
+    for (int e = 0; e < 16; e++) red[(wv * 16 + e) * 64 + l] = acc[e >> 2][e & 3];
+    __syncthreads();
+    for (int e = wv; e < 16; e += W) put(e >> 2, e & 3, spread_sum<W, 16>(red, e, l));
   }
 }
 
@@ -2005,8 +2047,8 @@ __global__ __launch_bounds__(64) void k_spread_mfma(int BnRun, long M1, long M2,
 // D[l / 16 + 4 r][l % 16], checked on the GPU against a host product).  The
 // products accumulate in FP64 in the matrix cores, so there is no carry.
 typedef double npme_d4 __attribute__((ext_vector_type(4)));
-template <int BN>
-__global__ __launch_bounds__(64) void k_spread_mfma64(int BnRun, long M1, long M2, long M3, int nt1,
+template <int BN, int W>
+__global__ __launch_bounds__(64 * W) void k_spread_mfma64(int BnRun, long M1, long M2, long M3, int nt1,
                                                       int nt2, int nt3,
                                                       const int *__restrict__ tileStart,
                                                       const int *__restrict__ tileList,
@@ -2018,7 +2060,10 @@ __global__ __launch_bounds__(64) void k_spread_mfma64(int BnRun, long M1, long M
   constexpr int TX = 16, TY = 8, TZ = 8;
   // one 16 KB block of rows, cleared per chunk by the wavefront in
   // contiguous runs (as in k_spread_mfma)
-  __shared__ __align__(16) double stage[64 * (TX + TY + TZ)];
+  constexpr int ROW = 64 * (TX + TY + TZ);
+  __shared__ __align__(16) double stages[W * ROW];
+  const int wv = W > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+  double *stage = stages + wv * ROW;
   double(*sA)[TX] = reinterpret_cast<double(*)[TX]>(stage);
   double(*sW2)[TY] = reinterpret_cast<double(*)[TY]>(stage + 64 * TX);
   double(*sW3)[TZ] = reinterpret_cast<double(*)[TZ]>(stage + 64 * (TX + TY));
@@ -2027,7 +2072,7 @@ __global__ __launch_bounds__(64) void k_spread_mfma64(int BnRun, long M1, long M
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   const int t3 = t % nt3, t2 = (t / nt3) % nt2, t1 = t / (nt3 * nt2);
   const int u1 = t1 * TX, u2 = t2 * TY, u3 = t3 * TZ;
-  const int l = threadIdx.x, n16 = l & 15, kq = l >> 4;
+  const int l = threadIdx.x & 63, n16 = l & 15, kq = l >> 4;
   const int beg = tileStart[t], end = tileStart[t + 1];
   int4 cm = make_int4(0, 0, 0, 0);
   double4 cf = make_double4(0, 0, 0, 0);
@@ -2040,9 +2085,9 @@ __global__ __launch_bounds__(64) void k_spread_mfma64(int BnRun, long M1, long M
       q = qre[c];
     }
   };
-  fetch(beg, cm, cf, cq);
+  fetch(beg + 64 * wv, cm, cf, cq);
   npme_d4 d0 = {0, 0, 0, 0}, d1 = d0, d2 = d0, d3 = d0;
-  for (int base = beg; base < end; base += 64) {
+  for (int base = beg + 64 * wv; base < end; base += 64 * W) {
     const int cnt = min(64, end - base);
     // row l as in k_spread_mfma: w2 stored (w2[0], w2[2], w2[4], w2[6],
     // w2[1], w2[3], w2[5], w2[7])
@@ -2074,8 +2119,8 @@ __global__ __launch_bounds__(64) void k_spread_mfma64(int BnRun, long M1, long M
       for (int j = 0; j < BA; j++)
         if (j < Bn && off + j >= 0 && off + j < TZ) sW3[l][off + j] = sh[j];
     }
-    __syncthreads();
-    fetch(base + 64, cm, cf, cq);
+    wave_lds_order();
+    fetch(base + 64 * W, cm, cf, cq);
     const int nstep = (cnt + 3) >> 2;  // rows past cnt are zero
     for (int st = 0; st < nstep; st++) {
       const int c = 4 * st + kq;
@@ -2087,82 +2132,79 @@ __global__ __launch_bounds__(64) void k_spread_mfma64(int BnRun, long M1, long M
       d2 = __builtin_amdgcn_mfma_f64_16x16x4f64(av, w2[2] * w3, d2, 0, 0, 0);
       d3 = __builtin_amdgcn_mfma_f64_16x16x4f64(av, w2[3] * w3, d3, 0, 0, 0);
     }
-    __syncthreads();  // the rows are rewritten by the next chunk
+    wave_lds_order();  // the rows are rewritten by the next chunk
   }
   const npme_d4 dd[4] = {d0, d1, d2, d3};
   const long p3 = u3 + (n16 & 7);
+  auto put = [&](int b, int r, double v) {
+    const long p2 = u2 + 2 * b + (n16 >> 3), p1 = u1 + kq + 4 * r;
+    if (p1 < M1 && p2 < M2 && p3 < M3) grid[(p1 * M2 + p2) * M3 + p3] = v;
+  };
+  if constexpr (W == 1) {
 #pragma unroll
-  for (int b = 0; b < 4; b++) {
-    const long p2 = u2 + 2 * b + (n16 >> 3);
+    for (int b = 0; b < 4; b++)
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const long p1 = u1 + kq + 4 * r;
-      if (p1 < M1 && p2 < M2 && p3 < M3) grid[(p1 * M2 + p2) * M3 + p3] = dd[b][r];
-    }
+      for (int r = 0; r < 4; r++) put(b, r, dd[b][r]);
+  } else {
+    double *red = stages;
+    __syncthreads();  // every wavefront is done with its rows
+#pragma unroll
+    for (int e = 0; e < 16; e++) red[(wv * 16 + e) * 64 + l] = dd[e >> 2][e & 3];
+    __syncthreads();
+    for (int e = wv; e < 16; e += W) put(e >> 2, e & 3, spread_sum<W, 16>(red, e, l));
   }
 }
 
+// wavefronts per spreading tile.  A tile's list is walked in chunks of 64
+// charges, ~8 us each (dependent loads, FP64 spline weights, LDS staging,
+// products), so with few tiles a launch is as long as its longest chain of
+// chunks: 22k charges on 96^3 (108 tiles of ~11 chunks) 76 -> 26 us, 1k charges
+// on 48^3 (18 tiles) 41 -> 15 us with several wavefronts a tile.  With
+// enough tiles one wavefront is best (the sums across wavefronts are extra):
+// the chip holds 4 wavefronts on each of its 1024 SIMDs.
+static int spread_waves(long tiles, size_t entries)
+{
+  const long chunks = (long)((entries + 63) / 64 + tiles - 1) / std::max(tiles, 1L);  // of a mean tile
+  int w = 1;
+  while (w < 4 && (long)w * 2 * tiles <= 4096 && 2 * w <= chunks + 1) w *= 2;
+  return w;
+}
+
 void launch_spread(bool fp64, bool complexK, long Bn, const long M[3], const int T[3],
-                   const int nt[3], const int *tileStart, const int *tileList, const void *qre,
+                   const int nt[3], const int *tileStart, const int *tileList, size_t entries, const void *qre,
                    const void *qim, const int4 *ms, const void *frac, void *grid, hipStream_t s)
 {
   const dim3 g((unsigned)(nt[0] * nt[1] * nt[2]));
-  if (!fp64 && !complexK && T[0] == 16 && T[1] == 8 && T[2] == 8) {
-#define NPME_SPREAD_M(BNV)                                                                      \
-  hipLaunchKernelGGL((k_spread_mfma<BNV>), g, dim3(64), 0, s, (int)Bn, M[0], M[1], M[2], nt[0],  \
-                     nt[1], nt[2], tileStart, tileList, (const float *)qre, ms,                 \
-                     (const float4 *)frac, (float *)grid)
-    switch (Bn) {
-      case 4: NPME_SPREAD_M(4); break;
-      case 6: NPME_SPREAD_M(6); break;
-      case 8: NPME_SPREAD_M(8); break;
-      case 10: NPME_SPREAD_M(10); break;
-      default: NPME_SPREAD_M(0); break;
-    }
-#undef NPME_SPREAD_M
-    NPME_HIP_CHECK(hipGetLastError());
-    return;
-  }
-  if (fp64 && !complexK && T[0] == 16 && T[1] == 8 && T[2] == 8) {
-#define NPME_SPREAD_M64(BNV)                                                                    \
-  hipLaunchKernelGGL((k_spread_mfma64<BNV>), g, dim3(64), 0, s, (int)Bn, M[0], M[1], M[2], nt[0],\
-                     nt[1], nt[2], tileStart, tileList, (const double *)qre, ms,                \
-                     (const double4 *)frac, (double *)grid)
-    switch (Bn) {
-      case 4: NPME_SPREAD_M64(4); break;
-      case 6: NPME_SPREAD_M64(6); break;
-      case 8: NPME_SPREAD_M64(8); break;
-      case 10: NPME_SPREAD_M64(10); break;
-      default: NPME_SPREAD_M64(0); break;
-    }
-#undef NPME_SPREAD_M64
-    NPME_HIP_CHECK(hipGetLastError());
-    return;
-  }
-  if (T[0] != 8 || T[1] != 8 || T[2] != 8) throw Error{NPME_ERR_UNSUPPORTED, "spreading tile shape"};
-#define NPME_SPREAD_B(R, CXV, BNV)                                                              \
-  hipLaunchKernelGGL((k_spread<R, CXV, BNV>), g, dim3(64), 0, s, (int)Bn, M[0], M[1], M[2],     \
-                     nt[0], nt[1], nt[2], tileStart, tileList, (const R *)qre, (const R *)qim,  \
-                     ms, (const typename V4t<R>::T *)frac, (R *)grid)
-#define NPME_SPREAD(R, CXV)                                                                     \
-  do {                                                                                          \
-    switch (Bn) {                                                                               \
-      case 4: NPME_SPREAD_B(R, CXV, 4); break;                                                  \
-      case 6: NPME_SPREAD_B(R, CXV, 6); break;                                                  \
-      case 8: NPME_SPREAD_B(R, CXV, 8); break;                                                  \
-      case 10: NPME_SPREAD_B(R, CXV, 10); break;                                                \
-      default: NPME_SPREAD_B(R, CXV, 0); break;                                                 \
-    }                                                                                           \
+  const int W = spread_waves((long)nt[0] * nt[1] * nt[2], entries);
+  const bool mfma = !complexK;  // 16 x 8 x 8 tiles on the matrix cores, else 8^3
+  if (T[0] != (mfma ? 16 : 8) || T[1] != 8 || T[2] != 8) throw Error{NPME_ERR_UNSUPPORTED, "spreading tile shape"};
+#define NPME_SPREAD_K(KERNEL, R, ...)                                                            \
+  hipLaunchKernelGGL(KERNEL, g, dim3(64 * W), 0, s, (int)Bn, M[0], M[1], M[2], nt[0], nt[1], nt[2], \
+                     tileStart, tileList, (const R *)qre, ##__VA_ARGS__, ms,                     \
+                     (const typename V4t<R>::T *)frac, (R *)grid)
+#define NPME_SPREAD_W(BNV, WV)                                                                   \
+  do {                                                                                           \
+    if (mfma && fp64) NPME_SPREAD_K((k_spread_mfma64<BNV, WV>), double);                         \
+    else if (mfma) NPME_SPREAD_K((k_spread_mfma<BNV, WV>), float);                               \
+    else if (fp64) NPME_SPREAD_K((k_spread<double, true, BNV, WV>), double, (const double *)qim);   \
+    else NPME_SPREAD_K((k_spread<float, true, BNV, WV>), float, (const float *)qim);             \
   } while (0)
-  if (fp64) {
-    if (complexK) NPME_SPREAD(double, true);
-    else NPME_SPREAD(double, false);
-  } else {
-    if (complexK) NPME_SPREAD(float, true);
-    else NPME_SPREAD(float, false);
+#define NPME_SPREAD_B(BNV)                                                                       \
+  do {                                                                                           \
+    if (W == 4) NPME_SPREAD_W(BNV, 4);                                                           \
+    else if (W == 2) NPME_SPREAD_W(BNV, 2);                                                      \
+    else NPME_SPREAD_W(BNV, 1);                                                                  \
+  } while (0)
+  switch (Bn) {
+    case 4: NPME_SPREAD_B(4); break;
+    case 6: NPME_SPREAD_B(6); break;
+    case 8: NPME_SPREAD_B(8); break;
+    case 10: NPME_SPREAD_B(10); break;
+    default: NPME_SPREAD_B(0); break;
   }
-#undef NPME_SPREAD
 #undef NPME_SPREAD_B
+#undef NPME_SPREAD_W
+#undef NPME_SPREAD_K
   NPME_HIP_CHECK(hipGetLastError());
 }
 
@@ -2334,8 +2376,10 @@ void launch_interp(bool fp64, bool complexK, long Bn, const long M[3], const dou
   const dim3 g((unsigned)(nt[0] * nt[1] * nt[2]));
   const int E = T + (int)Bn - 1;
   const size_t sh = (size_t)E * E * E * (fp64 ? 8 : 4) * (complexK ? 2 : 1);
+  // small blocks hold few charges and leave room for many workgroups a CU
+  const int threads = sh <= 8192 ? 64 : sh <= 16384 ? 128 : 256;
 #define NPME_INTERP_B(R, CXV, BNV)                                                              \
-  hipLaunchKernelGGL((k_interp_tile<R, CXV, BNV>), g, dim3(256), sh, s, (int)Bn, T, M[0], M[1],   \
+  hipLaunchKernelGGL((k_interp_tile<R, CXV, BNV>), g, dim3(threads), sh, s, (int)Bn, T, M[0], M[1],   \
                      M[2], nt[0], nt[1], nt[2], C[0], C[1], C[2], tileStart, tileList, ms,       \
                      (const typename V4t<R>::T *)frac, (const R *)grid, Vdir, perm, q_in,        \
                      fself[0], fself[1], Vout)
