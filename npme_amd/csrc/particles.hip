@@ -93,6 +93,16 @@ __device__ __forceinline__ void horner_fix_cx(const Real *c, Real r2, Real &re, 
   im = si;
 }
 
+// A wavefront's LDS accesses execute in program order, so words written by
+// some of its lanes and read by others need no barrier, only that the
+// compiler keeps the order.
+__device__ __forceinline__ void wave_lds_order()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ------------------------------------------------------------------ gather
 // charges in sorted order for the reciprocal sum (re and im in separate
 // arrays), so spreading does not read the direct sum's packed sources
@@ -1537,6 +1547,105 @@ __global__ __launch_bounds__(256) void k_cellpair_contact(DirectDev p, long ncel
   if (on) atomicOr(&flags[c * W + (o >> 5)], 1u << (o & 31));
 }
 
+// Stencils up to nNeigh = NLW_NN: a wavefront per cell.  The targets of a
+// cell share its flagged cells, so the wavefront enumerates their charges once
+// per batch of targets (counts scanned into LDS, each lane finding its charge
+// by a binary search), one charge per lane, 64 at a time, and evaluates them
+// against each target of the batch in turn; the lanes' FP64 sums are added
+// at the batch's end.  What bounds it is FP64 arithmetic (erfc and exp, ~200
+// instructions a pair): a thread per target, which chased cell, charge index
+// and charge through dependent loads with 1.5 wavefronts a SIMD, took 560 us
+// for 100k charges (~3e7 pairs), this 199 us.
+template <int KIND>
+__global__ __launch_bounds__(256) void k_direct_refpairs_cell(DirectDev p, long ncell, int W,
+                                                              const int2 *__restrict__ cellSE,
+                                                              const double4 *__restrict__ xs,
+                                                              const int *__restrict__ perm,
+                                                              const double *__restrict__ q,
+                                                              const unsigned *__restrict__ flags,
+                                                              double *__restrict__ Vdir)
+{
+  constexpr bool CX = kind_is_complex(KIND);
+  constexpr int NV = CX ? 8 : 4, TB = CX ? 2 : 4;  // values of a target, targets a batch
+  __shared__ int shStart[4][NLW_MAXC];
+  __shared__ int shPre[4][NLW_MAXC];
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const long c = (long)blockIdx.x * 4 + w;
+  if (c >= ncell) return;  // uniform per wavefront; no workgroup barrier below
+  const int2 home = cellSE[c];
+  if (home.y == 0) return;
+  const int hz = (int)(c % p.nb2), hy = (int)((c / p.nb2) % p.nb1), hx = (int)(c / ((long)p.nb1 * p.nb2));
+  const int nN = p.nNeigh, S = 2 * nN + 1, M = S * S * S;
+  int T = 0;
+  for (int c0 = 0; c0 < M; c0 += 64) {
+    const int o = c0 + lane;
+    int st = 0, cnt = 0;
+    // a flagged cell lies inside the grid
+    if (o < M && ((flags[c * W + (o >> 5)] >> (o & 31)) & 1u)) {
+      const int gx = hx + o / (S * S) - nN, gy = hy + (o / S) % S - nN, gz = hz + o % S - nN;
+      const int2 se = cellSE[((long)gx * p.nb1 + gy) * p.nb2 + gz];
+      st = se.x;
+      cnt = se.y;
+    }
+    int inc = cnt;
+    for (int k = 1; k < 64; k <<= 1) {
+      const int v = __shfl_up(inc, k);
+      if (lane >= k) inc += v;
+    }
+    if (o < M) {
+      shStart[w][o] = st;
+      shPre[w][o] = T + inc - cnt;
+    }
+    T += __shfl(inc, 63);
+  }
+  wave_lds_order();
+  for (int tb = 0; tb < home.y; tb += TB) {
+    const int mt = min(TB, home.y - tb), s0 = home.x + tb;
+    double part[TB][8];
+#pragma unroll
+    for (int i = 0; i < TB; i++)
+#pragma unroll
+      for (int k = 0; k < 8; k++) part[i][k] = 0;
+    for (int t0 = 0; t0 < T; t0 += 64) {
+      const int t = t0 + lane;
+      int j = -1;
+      double4 b = make_double4(0, 0, 0, 0);
+      double qr = 0, qim = 0;
+      if (t < T) {
+        unsigned ent;
+        j = nl_candidate(t, M, shStart[w], shPre[w], nullptr, 0, ent);
+        b = xs[j];
+        const size_t oj = (size_t)perm[j];
+        qr = CX ? q[2 * oj] : q[oj];
+        if (CX) qim = q[2 * oj + 1];
+      }
+#pragma unroll
+      for (int i = 0; i < TB; i++) {
+        if (i < mt) {  // uniform
+          const double4 me = xs[s0 + i];
+          const double rx = me.x - b.x, ry = me.y - b.y, rz = me.z - b.z;
+          if (j >= 0 && j != s0 + i)
+            pair_sr<double, KIND, 8>(p, rx, ry, rz, rx * rx + ry * ry + rz * rz, qr, qim, part[i], 0.0, 0.0);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TB; i++) {
+      if (i < mt) {
+        double mine = 0;
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+          double v = part[i][k];
+          for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+          if (lane == k) mine = v;
+        }
+        if (lane < NV) Vdir[(size_t)NV * (s0 + i) + lane] = mine;
+      }
+    }
+  }
+}
+
+// wider stencils: a thread per target
 template <int KIND>
 __global__ __launch_bounds__(256) void k_direct_refpairs(DirectDev p, size_t n, int W,
                                                          const int4 *__restrict__ cell,
@@ -1616,19 +1725,25 @@ void launch_direct_refpairs(const DirectParams &pp, size_t n, const int4 *cell, 
                             const unsigned *flags, double *Vdir, hipStream_t s)
 {
   const DirectDev d = refpair_dev(pp);
-  const dim3 g((unsigned)((n + 255) / 256));
   const int W = refpair_words(pp.nNeigh);
-  if (pp.kind == KIND_USER)
-    hipLaunchKernelGGL(k_direct_refpairs<KIND_USER>, g, dim3(256), 0, s, d, n, W, cell,
-                       (const int2 *)cellStart, xs, perm, q, flags, Vdir);
-  else if (pp.kind == KIND_USER_CX)
-    hipLaunchKernelGGL(k_direct_refpairs<KIND_USER_CX>, g, dim3(256), 0, s, d, n, W, cell,
-                       (const int2 *)cellStart, xs, perm, q, flags, Vdir);
-  else if (pp.kind == KIND_LAPLACE_ERF)
-    hipLaunchKernelGGL(k_direct_refpairs<KIND_LAPLACE_ERF>, g, dim3(256), 0, s, d, n, W, cell,
-                       (const int2 *)cellStart, xs, perm, q, flags, Vdir);
+  const long ncell = (long)pp.nb[0] * pp.nb[1] * pp.nb[2];
+  const bool cells = pp.nNeigh <= NLW_NN;
+  const int2 *cse = (const int2 *)cellStart;
+#define NPME_REFPAIRS(K)                                                                         \
+  do {                                                                                           \
+    if (cells)                                                                                   \
+      hipLaunchKernelGGL(k_direct_refpairs_cell<K>, dim3((unsigned)((ncell + 3) / 4)), dim3(256), 0, s, d, \
+                         ncell, W, cse, xs, perm, q, flags, Vdir);                               \
+    else                                                                                         \
+      hipLaunchKernelGGL(k_direct_refpairs<K>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, n, W, \
+                         cell, cse, xs, perm, q, flags, Vdir);                                   \
+  } while (0)
+  if (pp.kind == KIND_USER) NPME_REFPAIRS(KIND_USER);
+  else if (pp.kind == KIND_USER_CX) NPME_REFPAIRS(KIND_USER_CX);
+  else if (pp.kind == KIND_LAPLACE_ERF) NPME_REFPAIRS(KIND_LAPLACE_ERF);
   else
     throw Error{NPME_ERR_UNSUPPORTED, "no reference-pair direct sum for this kernel"};
+#undef NPME_REFPAIRS
   NPME_HIP_CHECK(hipGetLastError());
 }
 
@@ -1781,16 +1896,7 @@ constexpr int TS = 8;
 // W wavefronts share a tile: wavefront w takes the chunks w, w + W, ... of
 // its list, each with staging rows of its own, and the wavefronts' FP64 sums
 // are added in order at the end (spread_waves: sets whose tiles are too few
-// to fill the chip).  A wavefront's LDS accesses execute in program order, so
-// rows written by some of its lanes and read by others need no barrier, only
-// that the compiler keeps the order.
-__device__ __forceinline__ void wave_lds_order()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
+// to fill the chip).
 // the W wavefronts' sums of element e of lane l, added in order: red holds
 // [wavefront][E][64] doubles
 template <int W, int E> __device__ __forceinline__ double spread_sum(const double *red, int e, int l)
