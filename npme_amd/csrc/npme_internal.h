@@ -212,6 +212,13 @@ struct FFTPlan1D {
 };
 FFTPlan1D make_plan(int N);
 
+// host tables of one axis: twiddles exp(-2 pi i t / N) and the squared spline
+// factors |lambda|^2
+struct AxisTables {
+  long N = 0, Bn = 0;
+  std::vector<double> tw, lam;
+};
+
 // ------------------------------------------------------------- device state
 struct Handle;
 
@@ -337,6 +344,7 @@ struct Handle {
   double4 *d_xs = nullptr;       // [n] FP64 coordinates in sorted order (pair search)
   unsigned *d_cellFlags = nullptr;  // LaplaceOrig: interacting (cell, stencil offset) bits
   FFTPlan1D plan[3];
+  AxisTables axis[3];            // host tables of the grid sizes (grid_setup)
   size_t deviceBytes = 0;
   bool deviceSetup = false;      // per-charge set-up ran on the device
   bool fftPow8 = true;           // compile-time FFT kernels for N = 64, 512
@@ -402,12 +410,15 @@ struct GeoParams {
 // v on all three axes (wrapped int32 differences)
 bool sentinel_near_any(size_t n, const void *d_src, int4 v, int thr, hipStream_t s);
 void geometry_cells_device(const GeoParams &g, size_t n, const double *d_coord, int *d_perm,
-                           int4 *d_cellOf, int *d_cellSE, hipStream_t s);
+                           int4 *d_cellOf, int *d_cellSE, double4 *d_xs, hipStream_t s);
+// listSentinel: the list walk's padding source n must be away from every
+// charge; sentinelPlaced: it is
 void geometry_charges_device(const GeoParams &g, bool fp64, size_t n, const double *d_coord,
                              const int *d_perm, const int4 *d_cellOf, void *d_src, void *d_srcRes,
                              int4 *d_ms,
                              void *d_frac, DevBuf &tileStart, DevBuf &tileList, DevBuf &itileStart,
-                             DevBuf &itileList, size_t &nTileEntries, hipStream_t s);
+                             DevBuf &itileList, size_t &nTileEntries, bool listSentinel,
+                             bool &sentinelPlaced, hipStream_t s);
 // cell-row segments of the direct sum without a neighbour list, on the
 // device (segStart: nBlocks + 1 ints, nBlocks = ceil(n / 8)); returns their
 // number and the largest cluster offset (at least 1)

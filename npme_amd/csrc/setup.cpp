@@ -415,10 +415,8 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   h.d_perm = dalloc<int>(h, n);
   h.d_cell = dalloc<int4>(h, n);
   h.d_cellStart = dalloc<int>(h, 2 * (size_t)ncell);
-  geometry_cells_device(g, n, h.d_coordS, h.d_perm, h.d_cell, h.d_cellStart, s);
   h.d_xs = dalloc<double4>(h, n);
-  sorted_coords_device(n, h.d_perm, h.d_coordS, h.d_xs, s);
-  NPME_HIP_CHECK(hipStreamSynchronize(s));
+  geometry_cells_device(g, n, h.d_coordS, h.d_perm, h.d_cell, h.d_cellStart, h.d_xs, s);
   h.setupMs[2] = ms_since(t0);
 
   // direct-sum structure: the neighbour list (count, slice lengths and
@@ -473,16 +471,14 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   g.globalFrame = list ? 1 : 0;
   // [n + 1]: entry n is the neighbour list's zero-charge sentinel
   h.d_src = dalloc<char>(h, 4 * rs * (n + 1));
-  if (!f64) {
-    h.d_srcRes = dalloc<float4>(h, n + 1);
-    NPME_HIP_CHECK(hipMemsetAsync(static_cast<float4 *>(h.d_srcRes) + n, 0, sizeof(float4), s));
-  }
+  if (!f64) h.d_srcRes = dalloc<float4>(h, n + 1);
   h.d_frac = dalloc<char>(h, 4 * rs * n);
   h.d_ms = dalloc<int4>(h, n);
   DevBuf ts, tl, its, itl;
   size_t m = 0;
+  bool placed = false;
   geometry_charges_device(g, f64, n, h.d_coordS, h.d_perm, h.d_cell, h.d_src, h.d_srcRes, h.d_ms,
-                          h.d_frac, ts, tl, its, itl, m, s);
+                          h.d_frac, ts, tl, its, itl, m, list, placed, s);
   h.d_tileStart = (int *)adopt(h, ts);
   h.d_tileList = (int *)adopt(h, tl);
   h.nTileEntries = m;
@@ -498,8 +494,7 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   h.d_Vdir = dalloc<double>(h, vw * n);
   h.d_V = dalloc<double>(h, vw * n);
   h.d_qin = dalloc<double>(h, (h.complexK ? 2 : 1) * n);
-  NPME_HIP_CHECK(hipStreamSynchronize(s));
-  place_sentinel(h);
+  if (!placed) place_sentinel(h);
   h.setupMs[4] = ms_since(t0);
   return true;
 }
@@ -799,8 +794,18 @@ static void grid_setup(Handle &h)
   };
   size_t offTw[3], offTw64[3];
   for (int d = 0; d < 3; d++) {
-    h.plan[d] = make_plan((int)h.N[d]);
-    const std::vector<double> t = twiddles((int)h.N[d]);
+    // tables of the grid sizes and the spline order alone stay with the
+    // handle (their sines and cosines are ~0.1 ms of a 448^3 set-up)
+    AxisTables &ax = h.axis[d];
+    if (ax.N != h.N[d] || ax.Bn != h.Bn) {
+      h.plan[d] = make_plan((int)h.N[d]);
+      ax.tw = twiddles((int)h.N[d]);
+      ax.lam.resize(h.N[d]);
+      lambda2(h.N[d], h.Bn, ax.lam.data());
+      ax.N = h.N[d];
+      ax.Bn = h.Bn;
+    }
+    const std::vector<double> &t = ax.tw;
     offTw64[d] = put(t.data(), t.size() * sizeof(double));
     if (f64) {
       offTw[d] = offTw64[d];
@@ -859,11 +864,7 @@ static void grid_setup(Handle &h)
     const std::vector<double> tab = fulltrans_tables(h.N, h.ta, h.del, h.X, h.transD);
     const size_t offTab = put(tab.data(), tab.size() * sizeof(double));
     std::vector<double> lam;
-    for (int d = 0; d < 3; d++) {
-      std::vector<double> l(h.N[d]);
-      lambda2(h.N[d], h.Bn, l.data());
-      lam.insert(lam.end(), l.begin(), l.end());
-    }
+    for (int d = 0; d < 3; d++) lam.insert(lam.end(), h.axis[d].lam.begin(), h.axis[d].lam.end());
     const size_t offLam = put(lam.data(), lam.size() * sizeof(double));
     h.d_tables = dalloc<char>(h, blob.size());
     NPME_HIP_CHECK(hipMemcpyAsync(h.d_tables, blob.data(), blob.size(), hipMemcpyHostToDevice, h.stream));
@@ -927,11 +928,8 @@ static void grid_setup(Handle &h)
   // F: double per point for the real kernels, double2 for Helmholtz
   const size_t offTab = put(tab.data(), tab.size() * sizeof(double));
   std::vector<double> lam;
-  for (int d = 0; d < 3; d++) {
-    std::vector<double> l(h.N[d]);
-    lambda2(h.N[d], h.Bn, l.data());
-    lam.insert(lam.end(), l.begin(), l.begin() + Mf[d]);
-  }
+  for (int d = 0; d < 3; d++)
+    lam.insert(lam.end(), h.axis[d].lam.begin(), h.axis[d].lam.begin() + Mf[d]);
   const size_t offLam = put(lam.data(), lam.size() * sizeof(double));
   h.d_tables = dalloc<char>(h, blob.size());
   NPME_HIP_CHECK(hipMemcpyAsync(h.d_tables, blob.data(), blob.size(), hipMemcpyHostToDevice, h.stream));
