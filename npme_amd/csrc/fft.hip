@@ -1008,39 +1008,62 @@ __device__ __forceinline__ void rest8(T *lds, int c, int tj, const T *tw, T (*v)
   last8<T, L>(lds, c, tj, tw, v);
 }
 
-// passes B and D: column o * nInner + i, element n at o * outer + i * inner + n * pos
-template <typename Real, int L, bool HIN>
+// element r NB rows on from a thread's first one: the rows' offset is uniform
+// (scalar registers), the thread's own in 32 bits for FP32 (the passes bound
+// a column's elements to 2^31 over N / 2 rows, so N / 8 rows stay below 4 GB),
+// which costs no vector instruction per access; 64 bits for FP64
+template <typename Real> using LaneOff = typename std::conditional<sizeof(Real) == 4, unsigned, size_t>::type;
+template <typename T, typename O> __device__ __forceinline__ T *row_at(T *base, long rows, O lane)
+{
+  return reinterpret_cast<T *>(reinterpret_cast<char *>(base + rows) + lane);
+}
+template <typename T, typename O> __device__ __forceinline__ const T *row_at(const T *base, long rows, O lane)
+{
+  return reinterpret_cast<const T *>(reinterpret_cast<const char *>(base + rows) + lane);
+}
+
+// passes B (HIN: the first half of the rows non-zero, all stored) and D
+// (BACK: backward, the first half stored), and whole forward columns: column
+// o * nInner + i, element n at o * outer + i * inner + n * pos.  These passes
+// are bound by instruction issue rather than by HBM or LDS (512 points FP32:
+// smaller working sets that stay in the memory-side cache, or half the LDS
+// traffic with 16 x 32 points, are no faster), so direction and lengths are
+// template arguments and row offsets scalar: 643 -> 564 vector instructions
+// per 16 elements in B, none of them 64-bit multiplies, 86 -> 79 us at 512^3
+// (D 91 -> 89; FP64, bound by HBM, unchanged).
+template <typename Real, int L, bool HIN, bool BACK>
 __global__ __launch_bounds__(NT) void k_fft8_cols(CGeom g, const typename Cx<Real>::T *tw,
                                                   const typename Cx<Real>::T *__restrict__ in,
-                                                  typename Cx<Real>::T *__restrict__ out,
-                                                  int backward)
+                                                  typename Cx<Real>::T *__restrict__ out)
 {
   using T = typename Cx<Real>::T;
   using P = P8<L>;
   extern __shared__ char smem_raw[];
   T *lds = reinterpret_cast<T *>(smem_raw);
   const int c = threadIdx.x & (P::B - 1), tj = threadIdx.x >> P::LGB;
-  const int colg = (xcd_wg() << P::LGB) + c;
+  // the workgroup's first column (uniform) and this thread's
+  const int colg0 = xcd_wg() << P::LGB, colg = colg0 + c;
+  const int of = colg0 / g.nInner, inf = colg0 - of * g.nInner;
   const int o0 = colg / g.nInner;
   const bool valid = colg < g.nCols && colg - o0 * g.nInner < g.validInner;
-  const int o = valid ? o0 : 0, i = valid ? colg - o0 * g.nInner : 0;
+  // a column past the last takes the first one's place and is not stored
+  const int o = valid ? o0 : of, i = valid ? colg - o0 * g.nInner : inf;
+  using Off = LaneOff<Real>;
+  const T *src = in + ((long)of * g.inOuter + (long)inf * g.inInner);
+  T *dst = out + ((long)of * g.outOuter + (long)inf * g.outInner);
+  const Off sl = (Off)((o - of) * g.inOuter + (i - inf) * g.inInner + tj * g.inPos) * (Off)sizeof(T);
+  const Off dl = (Off)((o - of) * g.outOuter + (i - inf) * g.outInner + tj * g.outPos) * (Off)sizeof(T);
   const T *twl = twiddles8<T>(lds, lds_elems8<T, L>(), P::N, tw);
-  const T *src = in + ((long)o * g.inOuter + (long)i * g.inInner);
   T v[P::BPT][8];
 #pragma unroll
   for (int u = 0; u < P::BPT; u++) {
-    const int j = tj + u * P::TPC;
 #pragma unroll
     for (int r = 0; r < 8; r++) {
-      // the rows loaded are all below Lin (Lin = N, or N / 2 with HIN), and
-      // a column past the last reads column 0 and is not stored, so the
-      // loads need no condition and are all in flight together
-      const int n = j + r * P::NB;
       if (HIN && r >= 4) {
         v[u][r] = mk<T>(0, 0);
       } else {
-        const T x = src[(long)n * g.inPos];
-        v[u][r] = backward ? cconj(x) : x;
+        const T x = *row_at(src, (long)(u * P::TPC + r * P::NB) * g.inPos, sl);
+        v[u][r] = BACK ? cconj(x) : x;
       }
     }
   }
@@ -1048,15 +1071,11 @@ __global__ __launch_bounds__(NT) void k_fft8_cols(CGeom g, const typename Cx<Rea
   first8<T, L, HIN>(lds, c, tj, v);
   rest8<T, L>(lds, c, tj, twl, v);
   if (!valid) return;
-  T *dst = out + ((long)o * g.outOuter + (long)i * g.outInner);
 #pragma unroll
   for (int u = 0; u < P::BPT; u++) {
-    const int j = tj + u * P::TPC;
 #pragma unroll
-    for (int r = 0; r < 8; r++) {
-      const int n = j + r * P::NB;
-      if (n < g.Lout) dst[(long)n * g.outPos] = backward ? cconj(v[u][r]) : v[u][r];
-    }
+    for (int r = 0; r < (BACK ? 4 : 8); r++)
+      *row_at(dst, (long)(u * P::TPC + r * P::NB) * g.outPos, dl) = BACK ? cconj(v[u][r]) : v[u][r];
   }
 }
 
@@ -1075,9 +1094,12 @@ __global__ __launch_bounds__(NT) void k_fft8_conv(int nCols, int pos, int N2, in
   extern __shared__ char smem_raw[];
   T *lds = reinterpret_cast<T *>(smem_raw);
   const int c = threadIdx.x & (P::B - 1), tj = threadIdx.x >> P::LGB;
-  const int colg = (xcd_wg() << P::LGB) + c;
+  const int colg0 = xcd_wg() << P::LGB, colg = colg0 + c;
   const bool valid = colg < nCols && colg % C3 < Kv;
-  T *col = data + (valid ? colg : 0);
+  // a column past the last takes the first one's place and is not stored
+  using Off = LaneOff<Real>;
+  T *col = data + colg0;  // uniform; plus the thread's column and first row
+  const Off cl = ((Off)(valid ? c : 0) + (Off)tj * (Off)pos) * (Off)sizeof(T);
   const T *twl = twiddles8<T>(lds, lds_elems8<T, L>(), N, tw);
   // the G values of the thread's rows, fetched up front
   const GIndex gi = g_index<GM>(N, N2, Kv, N3fold, gfl, valid, colg, C3);
@@ -1093,9 +1115,8 @@ __global__ __launch_bounds__(NT) void k_fft8_conv(int nCols, int pos, int N2, in
       gv[u][r] = reinterpret_cast<const GT *>(Gv)[(long)g_a1<GM>(n, N, gfl) * 8 + gi.base];
       if constexpr (GM == 2)
         if (gfl & 8) gv[u][r] = cconj(gv[u][r]);
-      // rows below N / 2 hold data; an invalid column reads column 0 and is
-      // not stored, so the loads need no condition
-      v[u][r] = r < 4 ? col[(long)n * pos] : mk<T>(0, 0);
+      // rows below N / 2 hold data
+      v[u][r] = r < 4 ? *row_at(col, (long)(u * P::TPC + r * P::NB) * pos, cl) : mk<T>(0, 0);
     }
   }
   first8<T, L, true>(lds, c, tj, v);
@@ -1114,9 +1135,8 @@ __global__ __launch_bounds__(NT) void k_fft8_conv(int nCols, int pos, int N2, in
   if (!valid) return;
 #pragma unroll
   for (int u = 0; u < P::BPT; u++) {
-    const int j = tj + u * P::TPC;
 #pragma unroll
-    for (int r = 0; r < 4; r++) col[(long)(j + r * P::NB) * pos] = cconj(v[u][r]);
+    for (int r = 0; r < 4; r++) *row_at(col, (long)(u * P::TPC + r * P::NB) * pos, cl) = cconj(v[u][r]);
   }
 }
 
@@ -1293,19 +1313,20 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
   const int L8 = pow8 ? pow8_level(plan) : 0;
   // half the input: the pruned first stage (forward order: an even radix)
   const bool half = !backward && 2 * g.Lin == g.N;
-  if (!rows && L8 > 0 && (g.Lin == g.N || 2 * g.Lin == g.N) && g.Lout <= g.N) {
+  const bool half8 = 2 * g.Lin == g.N, full8 = g.Lin == g.N;
+  if (!rows && L8 > 0 && (backward ? full8 && 2 * g.Lout == g.N : (half8 || full8) && g.Lout == g.N)) {
     // N = 8^L: the compile-time kernel (4096 / N columns per workgroup)
     const dim3 grid((unsigned)((g.nCols + (4096 / g.N) - 1) / (4096 / g.N)));
     const size_t sh8 = pass_lds8(g.N, fp64);
-    const bool half8 = 2 * g.Lin == g.N;
-#define NPME_F8(R, LV, H)                                                                      \
-  hipLaunchKernelGGL((k_fft8_cols<R, LV, H>), grid, dim3(NT), sh8, s, c,                       \
+#define NPME_F8(R, LV, H, BK)                                                                  \
+  hipLaunchKernelGGL((k_fft8_cols<R, LV, H, BK>), grid, dim3(NT), sh8, s, c,                   \
                      (const typename Cx<R>::T *)tw, (const typename Cx<R>::T *)in,            \
-                     (typename Cx<R>::T *)out, (int)backward)
+                     (typename Cx<R>::T *)out)
 #define NPME_F8L(R, LV)                                                                        \
   do {                                                                                         \
-    if (half8) NPME_F8(R, LV, true);                                                           \
-    else NPME_F8(R, LV, false);                                                                \
+    if (backward) NPME_F8(R, LV, false, true);                                                 \
+    else if (half8) NPME_F8(R, LV, true, false);                                               \
+    else NPME_F8(R, LV, false, false);                                                         \
   } while (0)
     if (fp64) {
       if (L8 == 2) NPME_F8L(double, 2);
