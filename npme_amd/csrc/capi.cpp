@@ -505,6 +505,8 @@ int npme_print(const npme_handle *h, char *buf, size_t buflen)
     os << "  direct sum: the reference's interacting cell pairs, every point pair (FP64)\n";
   else if (H.useNlist)
     os << "  direct sum: neighbour list, " << H.nlistEntries << " entries\n";
+  else if (H.useFine)
+    os << "  direct sum: dense cells, " << H.nFineBlocks << " blocks of 64 charges\n";
   else
     os << "  direct sum: cell rows, " << H.nSegments << " segments\n";
   std::snprintf(buf, buflen, "%s", os.str().c_str());

@@ -944,6 +944,140 @@ void coord_bounds_device(size_t n, const double *d_coord, double mn[3], double m
   }
 }
 
+// ------------------------------------------------------------------ fine order
+// target blocks per cell (64 charges each)
+__global__ __launch_bounds__(256) void k_fine_count(long ncell, const int2 *__restrict__ cellSE,
+                                                    int *__restrict__ count)
+{
+  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c <= ncell) count[c] = c < ncell ? (cellSE[c].y + 63) / 64 : 0;
+}
+__global__ __launch_bounds__(256) void k_fine_blocks(long ncell, const int2 *__restrict__ cellSE,
+                                                     const int *__restrict__ blkStart, int2 *__restrict__ blk)
+{
+  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= ncell) return;
+  const int nb = (cellSE[c].y + 63) / 64;
+  for (int k = 0; k < nb; k++) blk[blkStart[c] + k] = make_int2((int)c, 64 * k);
+}
+// sort key: the first charge of the cell (cells keep their order), then the
+// Morton index of the position in the cell, 16 steps an axis
+__global__ __launch_bounds__(256) void k_fine_keys(size_t n, GeoParams g, const double4 *__restrict__ xs,
+                                                   const int4 *__restrict__ cellOf,
+                                                   const int2 *__restrict__ cellSE,
+                                                   unsigned long *__restrict__ key, int *__restrict__ idx)
+{
+  const size_t s = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const double4 x = xs[s];
+  const int4 c = cellOf[s];
+  const double v[3] = {x.x, x.y, x.z};
+  const int cc[3] = {c.x, c.y, c.z};
+  unsigned m = 0;
+  for (int d = 0; d < 3; d++) {
+    const double f = (v[d] - g.mn[d] - cc[d] * g.csB) / g.csB * 16.0;
+    const int b = min(max((int)f, 0), 15);
+    for (int k = 0; k < 4; k++) m |= (unsigned)((b >> k) & 1) << (3 * k + d);
+  }
+  const long cl = ((long)c.x * g.nb[1] + c.y) * g.nb[2] + c.z;
+  key[s] = ((unsigned long)cellSE[cl].x << 12) | m;
+  idx[s] = (int)s;
+}
+// per fine place: the charge, its source entry and residual
+__global__ __launch_bounds__(256) void k_fine_order(size_t n, const int *__restrict__ order,
+                                                    const int *__restrict__ perm, int *__restrict__ permF)
+{
+  const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (f < n) permF[f] = perm[order[f]];
+}
+template <typename V>
+__global__ __launch_bounds__(256) void k_fine_move(size_t n, const int *__restrict__ order,
+                                                   const V *__restrict__ in, V *__restrict__ out)
+{
+  const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (f <= n) out[f] = in[f < n ? (size_t)order[f] : n];
+}
+// bounding boxes of the groups of 16, relative to the cells' low corner and
+// widened by the rounding of positions of this extent to FP32
+__global__ __launch_bounds__(256) void k_fine_boxes(long nGroups, GeoParams g, float margin,
+                                                    const int2 *__restrict__ blk,
+                                                    const int2 *__restrict__ cellSE,
+                                                    const int *__restrict__ order,
+                                                    const double4 *__restrict__ xs, float4 *__restrict__ box)
+{
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nGroups) return;
+  const int2 b = blk[i / kFineSub];
+  const int2 se = cellSE[b.x];
+  const int k0 = b.y + kFineGroup * (int)(i % kFineSub), k1 = min(se.y, k0 + kFineGroup);
+  float lo[3] = {1e30f, 1e30f, 1e30f}, hi[3] = {-1e30f, -1e30f, -1e30f};  // empty: in reach of nothing
+  for (int k = k0; k < k1; k++) {
+    const double4 x = xs[order[se.x + k]];
+    const double v[3] = {x.x, x.y, x.z};
+    for (int d = 0; d < 3; d++) {
+      const float r = (float)(v[d] - g.mn[d]);
+      lo[d] = fminf(lo[d], r - margin);
+      hi[d] = fmaxf(hi[d], r + margin);
+    }
+  }
+  box[2 * i] = make_float4(lo[0], lo[1], lo[2], 0.f);
+  box[2 * i + 1] = make_float4(hi[0], hi[1], hi[2], 0.f);
+}
+
+int fine_blocks_device(const GeoParams &g, const int *d_cellSE, DevBuf &blkStart, hipStream_t s)
+{
+  const long ncell = (long)g.nb[0] * g.nb[1] * g.nb[2];
+  DevBuf cnt((ncell + 1) * sizeof(int));
+  blkStart.reset((ncell + 1) * sizeof(int));
+  hipLaunchKernelGGL(k_fine_count, grid_for(ncell + 1), dim3(256), 0, s, ncell, (const int2 *)d_cellSE,
+                     (int *)cnt.p);
+  NPME_HIP_CHECK(hipGetLastError());
+  exclusive_scan((const int *)cnt.p, (int *)blkStart.p, (size_t)ncell + 1, s);
+  int total = 0;
+  NPME_HIP_CHECK(hipMemcpyAsync(&total, (int *)blkStart.p + ncell, sizeof(int), hipMemcpyDeviceToHost, s));
+  NPME_HIP_CHECK(hipStreamSynchronize(s));
+  return total;
+}
+
+void fine_order_device(const GeoParams &g, size_t n, int nBlocks, const double4 *d_xs, const int4 *d_cellOf,
+                       const int *d_cellSE, const int *d_perm, const int *d_blkStart, int *d_order, int *d_permF,
+                       int2 *d_blk, float4 *d_box, hipStream_t s)
+{
+  const long ncell = (long)g.nb[0] * g.nb[1] * g.nb[2];
+  const int2 *cse = (const int2 *)d_cellSE;
+  DevBuf key(n * sizeof(unsigned long)), skey(n * sizeof(unsigned long)), idx(n * sizeof(int));
+  hipLaunchKernelGGL(k_fine_blocks, grid_for(ncell), dim3(256), 0, s, ncell, cse, d_blkStart, d_blk);
+  hipLaunchKernelGGL(k_fine_keys, grid_for(n), dim3(256), 0, s, n, g, d_xs, d_cellOf, cse,
+                     (unsigned long *)key.p, (int *)idx.p);
+  NPME_HIP_CHECK(hipGetLastError());
+  sort_pairs((const unsigned long *)key.p, (unsigned long *)skey.p, (const int *)idx.p, d_order, n,
+             key_bits(((unsigned long)n << 12) | 4095), s);
+  hipLaunchKernelGGL(k_fine_order, grid_for(n), dim3(256), 0, s, n, d_order, d_perm, d_permF);
+  double extent = 0;
+  for (int d = 0; d < 3; d++) extent = std::max(extent, g.nb[d] * g.csB);
+  const long ng = (long)kFineSub * nBlocks;
+  hipLaunchKernelGGL(k_fine_boxes, grid_for(ng), dim3(256), 0, s, ng, g, (float)(4.0e-7 * extent), d_blk, cse,
+                     d_order, d_xs, d_box);
+  NPME_HIP_CHECK(hipGetLastError());
+  NPME_HIP_CHECK(hipStreamSynchronize(s));  // before the scratch returns to the pool
+}
+
+void fine_sources_device(bool fp64, size_t n, const int *d_order, const void *srcS, const void *resS, void *src,
+                         void *res, hipStream_t s)
+{
+  if (fp64) {
+    hipLaunchKernelGGL(k_fine_move<double4>, grid_for(n + 1), dim3(256), 0, s, n, d_order,
+                       (const double4 *)srcS, (double4 *)src);
+  } else {
+    hipLaunchKernelGGL(k_fine_move<float4>, grid_for(n + 1), dim3(256), 0, s, n, d_order, (const float4 *)srcS,
+                       (float4 *)src);
+    hipLaunchKernelGGL(k_fine_move<float4>, grid_for(n + 1), dim3(256), 0, s, n, d_order, (const float4 *)resS,
+                       (float4 *)res);
+  }
+  NPME_HIP_CHECK(hipGetLastError());
+  NPME_HIP_CHECK(hipStreamSynchronize(s));  // before the sorted copies return to the pool
+}
+
 void sorted_coords_device(size_t n, const int *d_perm, const double *d_coord, double4 *d_xs,
                           hipStream_t s)
 {

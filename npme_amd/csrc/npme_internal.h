@@ -325,6 +325,12 @@ struct Handle {
   int4 *d_ms = nullptr;          // [n] stencil start u0 per dim (u = m + N/4)
   void *d_frac = nullptr;        // [n] float4/double4 fractional spline arguments
   int *d_tileStart = nullptr;    // [ntiles + 1]
+  // direct sum of densely packed charges (k_direct_fine)
+  bool useFine = false;
+  int nFineBlocks = 0;
+  int *d_fineOrder = nullptr, *d_finePerm = nullptr, *d_fineStart = nullptr;
+  int2 *d_fineBlk = nullptr;
+  float4 *d_fineBox = nullptr;
   int *d_tileList = nullptr;     // [nlist]
   size_t nTileEntries = 0;       // its length
   int TI = 16;                   // interpolation tile edge
@@ -419,6 +425,24 @@ void geometry_charges_device(const GeoParams &g, bool fp64, size_t n, const doub
                              void *d_frac, DevBuf &tileStart, DevBuf &tileList, DevBuf &itileStart,
                              DevBuf &itileList, size_t &nTileEntries, bool listSentinel,
                              bool &sentinelPlaced, hipStream_t s);
+// fine order of densely packed charges (k_direct_fine): blocks of 64 charges
+// of one cell in kFineSub groups of kFineGroup
+constexpr int kFineGroup = 16, kFineSub = 64 / kFineGroup;
+struct FineDev {
+  int nBlocks;
+  const int2 *blk, *cellSE;  // per block (cell, first charge in it); (start, count) of every cell
+  const int *blkStart;       // first block of every cell
+  const float4 *box;         // (low, high) corners of every group
+  const int *order;          // sorted index of every fine place
+};
+// blocks of every cell (scanned); returns their number
+int fine_blocks_device(const GeoParams &g, const int *d_cellSE, DevBuf &blkStart, hipStream_t s);
+void fine_order_device(const GeoParams &g, size_t n, int nBlocks, const double4 *d_xs, const int4 *d_cellOf,
+                       const int *d_cellSE, const int *d_perm, const int *d_blkStart, int *d_order, int *d_permF,
+                       int2 *d_blk, float4 *d_box, hipStream_t s);
+// sources (and residuals) from sorted to fine order
+void fine_sources_device(bool fp64, size_t n, const int *d_order, const void *srcS, const void *resS, void *src,
+                         void *res, hipStream_t s);
 // cell-row segments of the direct sum without a neighbour list, on the
 // device (segStart: nBlocks + 1 ints, nBlocks = ceil(n / 8)); returns their
 // number and the largest cluster offset (at least 1)
@@ -550,6 +574,10 @@ void launch_gather_q(bool fp64, bool complexK, size_t n, const int *perm, const 
 // packed source charges (src[s].w, qi) and the spreading copy (qre, qim)
 void launch_gather_both(bool fp64, bool complexK, size_t n, const int *perm, const double *q_in,
                         void *src, void *qi, void *qre, void *qim, hipStream_t s);
+void launch_gather_src(bool fp64, bool complexK, size_t n, const int *perm, const double *q_in, void *src,
+                       void *qi, hipStream_t s);
+void launch_direct_fine(bool fp64, const DirectParams &p, const FineDev &g, const void *src, const void *res,
+                        const void *qi, double *Vdir, hipStream_t s);
 void launch_direct(bool fp64, const DirectParams &p, size_t n, const void *src, const void *res,
                    const void *qi, const int4 *cell, const int *segStart, const void *segs, int nP, double csA,
                    double *Vdir, hipStream_t s);

@@ -144,6 +144,36 @@ __global__ void k_gather_both(size_t n, const int *__restrict__ perm, const doub
   }
 }
 
+// the direct sum's packed source charges alone, in an order of their own
+template <typename Real, bool CX>
+__global__ void k_gather_src(size_t n, const int *__restrict__ perm, const double *__restrict__ q,
+                             typename V4t<Real>::T *__restrict__ src, Real *__restrict__ qi)
+{
+  const size_t s = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const size_t o = (size_t)perm[s];
+  src[s].w = (Real)q[CX ? 2 * o : o];
+  if (CX) qi[s] = (Real)q[2 * o + 1];
+}
+
+void launch_gather_src(bool fp64, bool complexK, size_t n, const int *perm, const double *q_in, void *src,
+                       void *qi, hipStream_t s)
+{
+  const dim3 grid((unsigned)((n + 255) / 256));
+#define NPME_GS(R, CXV)                                                                        \
+  hipLaunchKernelGGL((k_gather_src<R, CXV>), grid, dim3(256), 0, s, n, perm, q_in,              \
+                     (typename V4t<R>::T *)src, (R *)qi)
+  if (fp64) {
+    if (complexK) NPME_GS(double, true);
+    else NPME_GS(double, false);
+  } else {
+    if (complexK) NPME_GS(float, true);
+    else NPME_GS(float, false);
+  }
+#undef NPME_GS
+  NPME_HIP_CHECK(hipGetLastError());
+}
+
 void launch_gather_both(bool fp64, bool complexK, size_t n, const int *perm, const double *q_in,
                         void *src, void *qi, void *qre, void *qim, hipStream_t s)
 {
@@ -1447,6 +1477,238 @@ void launch_direct_nl(bool fp64, const DirectParams &p, size_t n, const void *sr
   }
 #undef NPME_DNL
 #undef NPME_DNL_D
+  NPME_HIP_CHECK(hipGetLastError());
+}
+
+// ------------------------------------------------------------------ dense cells
+// Direct sum without a list for densely packed charges (thousands per cell,
+// too many pairs to list).  The charges of a cell are ordered along a Morton
+// curve inside it ("fine" order), so 64 consecutive ones, a target block (one
+// target per lane), and 16 consecutive ones, a source group, are compact, and
+// each group has a bounding box.  A workgroup of 4 wavefronts takes a target
+// block: its wavefronts share the groups of the block's cell stencil, test
+// their boxes against the block's 64 at a time, and walk the groups in reach
+// source by source.  A source is wave-uniform (scalar loads), every lane
+// pairs its target with it; groups wholly inside the cutoff of all targets
+// need no test, in the others a source that reaches no lane is skipped.
+// Positions are in the list walk's frame (the wrapped int32 differences are
+// exact: stencil neighbours are less than 2 clusters apart).  FP32 sums of a
+// group carry into FP64.  The cell-row walk pairs every target of a block of
+// 8 with all charges of the cell rows in reach, 3.7 candidates per pair
+// inside the cutoff at 4 A cells against ~1.6 here: 4M charges in 64 Gaussian
+// blobs (7e10 pairs) 181 -> 81 ms, bound by the ~37 instructions of a pair.
+template <typename Real, int KIND, bool FIXP, int MAXD>
+__global__ __launch_bounds__(256) void k_direct_fine(DirectDev p, FineDev g,
+                                                     const typename V4t<Real>::T *__restrict__ src,
+                                                     const float4 *__restrict__ res,
+                                                     const Real *__restrict__ qi, double *__restrict__ Vdir)
+{
+  using V4 = typename V4t<Real>::T;
+  constexpr bool CX = pair_is_complex(KIND);
+  constexpr int NV = CX ? 8 : 4;
+  __shared__ int shSub[NLW_MAXC], shPre[NLW_MAXC], shFirst[NLW_MAXC], shCnt[NLW_MAXC];
+  __shared__ int shT;
+  __shared__ double red[3][NV][64];
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int2 blk = g.blk[b];  // cell, first charge of the block within it
+  const int2 home = g.cellSE[blk.x];
+  const int f0 = home.x + blk.y, ft = f0 + lane;
+  const bool tvalid = blk.y + lane < home.y;
+  const int hz = blk.x % p.nb2, hy = (blk.x / p.nb2) % p.nb1, hx = blk.x / (p.nb2 * p.nb1);
+  const int nN = p.nNeigh, S = 2 * nN + 1, M = S * S * S;
+  if (w == 0) {  // the stencil's groups as one sequence
+    int T = 0;
+    for (int c0 = 0; c0 < M; c0 += 64) {
+      const int o = c0 + lane;
+      int cnt = 0, first = 0, sub = 0;
+      if (o < M) {
+        const int gx = hx + o / (S * S) - nN, gy = hy + (o / S) % S - nN, gz = hz + o % S - nN;
+        if (gx >= 0 && gy >= 0 && gz >= 0 && gx < p.nb0 && gy < p.nb1 && gz < p.nb2) {
+          const int c = (gx * p.nb1 + gy) * p.nb2 + gz;
+          const int2 se = g.cellSE[c];
+          first = se.x;
+          cnt = se.y;
+          sub = kFineSub * g.blkStart[c];
+        }
+      }
+      const int ng = (cnt + kFineGroup - 1) / kFineGroup;
+      int inc = ng;
+      for (int k = 1; k < 64; k <<= 1) {
+        const int v = __shfl_up(inc, k);
+        if (lane >= k) inc += v;
+      }
+      if (o < M) {
+        shSub[o] = sub;
+        shFirst[o] = first;
+        shCnt[o] = cnt;
+        shPre[o] = T + inc - ng;
+      }
+      T += __shfl(inc, 63);
+    }
+    if (lane == 0) shT = T;
+  }
+  // the block's box: the union of its groups'
+  float tl[3], th[3];
+  {
+    float4 lo = g.box[2 * (kFineSub * b)], hi = g.box[2 * (kFineSub * b) + 1];
+    for (int k = 1; k < kFineSub; k++) {
+      const float4 l2 = g.box[2 * (kFineSub * b + k)], h2 = g.box[2 * (kFineSub * b + k) + 1];
+      lo = make_float4(fminf(lo.x, l2.x), fminf(lo.y, l2.y), fminf(lo.z, l2.z), 0.f);
+      hi = make_float4(fmaxf(hi.x, h2.x), fmaxf(hi.y, h2.y), fmaxf(hi.z, h2.z), 0.f);
+    }
+    tl[0] = lo.x, tl[1] = lo.y, tl[2] = lo.z;
+    th[0] = hi.x, th[1] = hi.y, th[2] = hi.z;
+  }
+  const V4 me = src[tvalid ? ft : f0];
+  int mx = 0, my = 0, mz = 0;
+  float4 mres = make_float4(0, 0, 0, 0);
+  if constexpr (FIXP) {
+    mx = __float_as_int(me.x);
+    my = __float_as_int(me.y);
+    mz = __float_as_int(me.z);
+    mres = res[tvalid ? ft : f0];
+  }
+  const Real R2 = (Real)(p.Rdir * p.Rdir);
+  const Real u2 = (Real)(p.fxInvD * p.fxInvD);
+  // group decisions keep a margin to the pair test (the boxes are widened by
+  // the rounding of their positions)
+  const float Rn2 = (float)(p.Rdir * p.Rdir * (1.0 + 1.0e-6)), Rf2 = (float)(p.Rdir * p.Rdir * (1.0 - 1.0e-6));
+  Real topA = coef_a<Real>(p)[2 * MAXD], topB = coef_b<Real>(p)[2 * MAXD];
+  asm volatile("" : "+v"(topA), "+v"(topB));  // held in VGPRs for the pair loop
+  double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  __syncthreads();
+  const int T = shT;
+  for (int t0 = 64 * w; t0 < T; t0 += 256) {
+    const int t = t0 + lane;
+    bool hit = false, full = false;
+    int first = 0, cnt = 0;
+    if (t < T) {
+      int lo = 0, hi = M - 1;  // last cell whose first group is at or before t
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (shPre[mid] <= t) lo = mid;
+        else hi = mid - 1;
+      }
+      const int k = t - shPre[lo];
+      first = shFirst[lo] + kFineGroup * k;
+      cnt = min(kFineGroup, shCnt[lo] - kFineGroup * k);
+      const float4 bl = g.box[2 * (shSub[lo] + k)], bh = g.box[2 * (shSub[lo] + k) + 1];
+      const float sl[3] = {bl.x, bl.y, bl.z}, sh[3] = {bh.x, bh.y, bh.z};
+      float n2 = 0, f2 = 0;
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        const float a = fmaxf(0.f, fmaxf(sl[d] - th[d], tl[d] - sh[d]));
+        const float c = fmaxf(sh[d] - tl[d], th[d] - sl[d]);
+        n2 += a * a;
+        f2 += c * c;
+      }
+      hit = n2 < Rn2;
+      // the block's own charges take the tested path, which skips the target
+      full = f2 < Rf2 && (first < f0 || first >= f0 + 64);
+    }
+    unsigned long long todo = __ballot(hit);
+    const unsigned long long fulls = __ballot(full);
+    while (todo) {  // uniform
+      const int l = __ffsll((unsigned long long)todo) - 1;
+      todo &= todo - 1;
+      const int j0 = __builtin_amdgcn_readlane(first, l), nj = __builtin_amdgcn_readlane(cnt, l);
+      const bool all = (fulls >> l) & 1ull;
+      Real part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      auto pair = [&](int j, bool tested) {
+        const V4 o = src[j];  // uniform
+        Real rx, ry, rz, r2;
+        if constexpr (FIXP) {
+          const int dx = mx - __float_as_int(o.x), dy = my - __float_as_int(o.y), dz = mz - __float_as_int(o.z);
+          rx = (Real)dx;
+          ry = (Real)dy;
+          rz = (Real)dz;
+          r2 = rx * rx + ry * ry + rz * rz;
+          if (__builtin_amdgcn_ballot_w64(r2 < (Real)p.fxClose2u)) {  // rare, uniform
+            if (r2 < (Real)p.fxClose2u) {
+              const float4 ro = res[j];
+              rx = (Real)dx + (mres.x - ro.x);
+              ry = (Real)dy + (mres.y - ro.y);
+              rz = (Real)dz + (mres.z - ro.z);
+              r2 = rx * rx + ry * ry + rz * rz;
+            }
+          }
+          r2 = r2 * u2;
+        } else {
+          rx = me.x - o.x;
+          ry = me.y - o.y;
+          rz = me.z - o.z;
+          r2 = rx * rx + ry * ry + rz * rz;
+        }
+        Real qr = o.w, qim = CX ? qi[j] : (Real)0;
+        if (tested) {
+          const bool in = r2 < R2 && j != ft;
+          if (!__builtin_amdgcn_ballot_w64(in)) return;  // uniform
+          r2 = in ? r2 : R2;
+          qr = in ? qr : (Real)0;
+          if (CX) qim = in ? qim : (Real)0;
+        }
+        pair_sr<Real, KIND, MAXD>(p, rx, ry, rz, r2, qr, qim, part, topA, topB);
+      };
+      if (all) {
+        if (nj == kFineGroup) {
+#pragma unroll 4
+          for (int k = 0; k < kFineGroup; k++) pair(j0 + k, false);
+        } else {
+          for (int k = 0; k < nj; k++) pair(j0 + k, false);
+        }
+      } else {
+        for (int k = 0; k < nj; k++) pair(j0 + k, true);
+      }
+#pragma unroll
+      for (int c = 0; c < NV; c++) acc[c] += (double)part[c];
+    }
+  }
+  // the wavefronts' sums, added in order
+  if (w > 0) {
+#pragma unroll
+    for (int c = 0; c < NV; c++) red[w - 1][c][lane] = acc[c];
+  }
+  __syncthreads();
+  if (w > 0 || !tvalid) return;
+  const size_t s = (size_t)g.order[ft];
+#pragma unroll
+  for (int c = 0; c < NV; c++) {
+    double v = acc[c] + red[0][c][lane] + red[1][c][lane] + red[2][c][lane];
+    if (FIXP && c >= (CX ? 2 : 1)) v *= p.fxInvD;  // from fixed-point units to lengths
+    Vdir[NV * s + c] = v;
+  }
+}
+
+void launch_direct_fine(bool fp64, const DirectParams &p, const FineDev &g, const void *src, const void *res,
+                        const void *qi, double *Vdir, hipStream_t s)
+{
+  const DirectDev d = direct_dev(p);
+#define NPME_DF_D(R, K, HL, D)                                                                  \
+  hipLaunchKernelGGL((k_direct_fine<R, K, HL, D>), dim3((unsigned)g.nBlocks), dim3(256), 0, s, d, g, \
+                     (const typename V4t<R>::T *)src, (const float4 *)res, (const R *)qi, Vdir)
+#define NPME_DF(R, K, HL)                                                                       \
+  do {                                                                                          \
+    if (p.Nder <= 4) NPME_DF_D(R, K, HL, 4);                                                    \
+    else if (p.Nder <= 6) NPME_DF_D(R, K, HL, 6);                                               \
+    else if (p.Nder <= 8) NPME_DF_D(R, K, HL, 8);                                               \
+    else if (p.Nder <= 16) NPME_DF_D(R, K, HL, 16);                                             \
+    else NPME_DF_D(R, K, HL, 30);                                                               \
+  } while (0)
+  const int kind = fp64 ? p.kind : pair_kind32(p);
+  if (fp64) {
+    if (kind == KIND_LAPLACE) NPME_DF(double, KIND_LAPLACE, false);
+    else if (kind == KIND_RALPHA) NPME_DF(double, KIND_RALPHA, false);
+    else NPME_DF(double, KIND_HELMHOLTZ, false);
+  } else {
+    if (kind == KIND_LAPLACE) NPME_DF(float, KIND_LAPLACE, true);
+    else if (kind == KIND_RALPHA_HALF) NPME_DF(float, KIND_RALPHA_HALF, true);
+    else if (kind == KIND_RALPHA) NPME_DF(float, KIND_RALPHA, true);
+    else if (kind == KIND_HELMHOLTZ_REAL) NPME_DF(float, KIND_HELMHOLTZ_REAL, true);
+    else NPME_DF(float, KIND_HELMHOLTZ, true);
+  }
+#undef NPME_DF
+#undef NPME_DF_D
   NPME_HIP_CHECK(hipGetLastError());
 }
 

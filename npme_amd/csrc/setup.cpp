@@ -64,7 +64,8 @@ void handle_free_device(Handle &h, bool keepG)
                   h.d_sliceStart, h.d_sliceLen, h.d_qi, h.d_cell, h.d_cellStart, h.d_ms, h.d_frac,
                   h.d_tileStart, h.d_tileList, h.d_grid, h.d_buf1, h.d_buf2,
                   h.d_tables, h.d_Vdir, h.d_V, h.d_qin, h.d_coordS, h.d_xs,
-                  h.d_qs, h.d_qsi, h.d_utab, h.d_cellFlags};
+                  h.d_qs, h.d_qsi, h.d_utab, h.d_cellFlags, h.d_fineOrder, h.d_finePerm, h.d_fineStart,
+                  h.d_fineBlk, h.d_fineBox};
   // queued work of this handle may still read its buffers
   if (h.stream) (void)hipStreamSynchronize(h.stream);
   if (h.stream2) (void)hipStreamSynchronize(h.stream2);
@@ -97,6 +98,11 @@ void handle_free_device(Handle &h, bool keepG)
   h.d_xs = nullptr;
   h.d_utab = nullptr;
   h.d_cellFlags = nullptr;
+  h.d_fineOrder = h.d_finePerm = h.d_fineStart = nullptr;
+  h.d_fineBlk = nullptr;
+  h.d_fineBox = nullptr;
+  h.useFine = false;
+  h.nFineBlocks = 0;
   h.coordStaged = h.stagedBoundsReady = false;
   h.deviceBytes = h.d_G ? h.gBytes : 0;
 }
@@ -452,7 +458,27 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   }
   int maxOff = 1;
   h.nSegments = 0;
-  if (!list) {
+  // without a list: the fine order when the blocks of 64 charges of one cell
+  // are at least half full on average (sparser cells leave its lanes idle,
+  // where the cell rows' blocks of 8 do not) and the stencil's differences fit
+  // the list's frame, else the cell rows
+  if (!list && !h.trans && !kind_ref_pairs(h.ker.kind) && h.nNeigh <= 3 && h.nNeigh + 1 < 2 * h.nCellClust1D) {
+    DevBuf start;
+    const int nb = fine_blocks_device(g, h.d_cellStart, start, s);
+    if (n >= 32 * (size_t)nb) {
+      h.useFine = true;
+      h.nFineBlocks = nb;
+      h.d_fineStart = (int *)adopt(h, start);
+      h.d_fineOrder = dalloc<int>(h, n);
+      h.d_finePerm = dalloc<int>(h, n);
+      h.d_fineBlk = dalloc<int2>(h, nb);
+      h.d_fineBox = dalloc<float4>(h, 2 * kFineSub * (size_t)nb);
+      fine_order_device(g, n, nb, h.d_xs, h.d_cell, h.d_cellStart, h.d_perm, h.d_fineStart, h.d_fineOrder,
+                        h.d_finePerm, h.d_fineBlk, h.d_fineBox, s);
+    }
+  }
+  const bool frame = list || h.useFine;  // positions in one frame
+  if (!frame) {
     const long nBlocks = ((long)n + 7) / 8;
     h.d_segStart = dalloc<int>(h, nBlocks + 1);
     DevBuf segs;
@@ -465,10 +491,10 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   // positions, spline windows and tile lists; the fixed-point scale
   // depends on how far the direct sum's sources reach (list: the adjacent
   // clusters)
-  h.fxShift = list ? kListShift : fixed_shift(maxOff);
+  h.fxShift = frame ? kListShift : fixed_shift(maxOff);
   g.fxShift = h.fxShift;
   g.fxScale = std::ldexp(1.0, h.fxShift) / h.csA;
-  g.globalFrame = list ? 1 : 0;
+  g.globalFrame = frame ? 1 : 0;
   // [n + 1]: entry n is the neighbour list's zero-charge sentinel
   h.d_src = dalloc<char>(h, 4 * rs * (n + 1));
   if (!f64) h.d_srcRes = dalloc<float4>(h, n + 1);
@@ -477,8 +503,15 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   DevBuf ts, tl, its, itl;
   size_t m = 0;
   bool placed = false;
-  geometry_charges_device(g, f64, n, h.d_coordS, h.d_perm, h.d_cell, h.d_src, h.d_srcRes, h.d_ms,
+  DevBuf srcS, resS;  // sorted order, moved to the fine order below
+  if (h.useFine) {
+    srcS.reset(4 * rs * (n + 1));
+    resS.reset(sizeof(float4) * (n + 1));
+  }
+  geometry_charges_device(g, f64, n, h.d_coordS, h.d_perm, h.d_cell, h.useFine ? srcS.p : h.d_src,
+                          h.useFine ? resS.p : h.d_srcRes, h.d_ms,
                           h.d_frac, ts, tl, its, itl, m, list, placed, s);
+  if (h.useFine) fine_sources_device(f64, n, h.d_fineOrder, srcS.p, resS.p, h.d_src, h.d_srcRes, s);
   h.d_tileStart = (int *)adopt(h, ts);
   h.d_tileList = (int *)adopt(h, tl);
   h.nTileEntries = m;
@@ -1364,7 +1397,10 @@ static void calcv_launches(Handle &h, const double *d_q, double *d_Vout, bool sp
   // sum's packed sources and the spreading copy (a box pair has no direct
   // sum, so only the spreading copy)
   auto gather = [&] {
-    if (doDirect)
+    if (h.useFine) {
+      launch_gather_src(f64, cx, h.n, h.d_finePerm, d_q, h.d_src, h.d_qi, s);
+      launch_gather_q(f64, cx, h.n, h.d_perm, d_q, h.d_qs, h.d_qsi, s);
+    } else if (doDirect)
       launch_gather_both(f64, cx, h.n, h.d_perm, d_q, h.d_src, h.d_qi, h.d_qs, h.d_qsi, s);
     else
       launch_gather_q(f64, cx, h.n, h.d_perm, d_q, h.d_qs, h.d_qsi, s);
@@ -1373,6 +1409,11 @@ static void calcv_launches(Handle &h, const double *d_q, double *d_Vout, bool sp
     if (refPairs)
       launch_direct_refpairs(dp, h.n, h.d_cell, h.d_cellStart, h.d_xs, h.d_perm, d_q, h.d_cellFlags,
                              h.d_Vdir, ds);
+    else if (h.useFine)
+      launch_direct_fine(f64, dp,
+                         FineDev{h.nFineBlocks, h.d_fineBlk, (const int2 *)h.d_cellStart, h.d_fineStart, h.d_fineBox,
+                                 h.d_fineOrder},
+                         h.d_src, h.d_srcRes, h.d_qi, h.d_Vdir, ds);
     else if (h.useNlist)
       launch_direct_nl(f64, dp, h.n, h.d_src, h.d_srcRes, h.d_qi, h.d_sliceStart, h.d_sliceLen,
                        h.d_nlist, h.csA, h.d_Vdir, ds);
