@@ -31,9 +31,11 @@
 // 8/4/2/7/5/3, a separate LDS fill, LDS drain and G pass, ~170 VGPRs, 4096
 // values a workgroup whatever the length, so 2 to 4 adjacent columns at
 // lengths near 1000) took, FP32, passes A/B/C/D/E: 32/60/96/56/31 us on 256 x
-// 384 x 500 (now 24/34/58/37/25: 4.4 TB/s in B), 79/124/558/119/77 on 320 x
-// 320 x 1152 (now 50/92/212/91/60), 42/85/342/80/41 on 448^3 (now
-// 37/68/157/68/45); FP64 120^3 15/14/23/13/14 (now 10/10/14/10/9).
+// 384 x 500 (now 25/34/56/34/25: 4.4 TB/s in B), 79/124/558/119/77 on 320 x
+// 320 x 1152 (now 51/90/201/89/58), 42/85/342/80/41 on 448^3 (now
+// 38/65/149/68/43); FP64 120^3 15/14/23/13/14 (now 9/9/13/9/9).  Directions and
+// lengths are template arguments: conditions on every stored element had
+// cost passes C and D 3 to 9%.
 // N = 64 and 512 have kernels of their own (below) with every index a
 // compile-time constant.
 #include <type_traits>
@@ -509,8 +511,9 @@ template <typename T, int R> __device__ __forceinline__ void last_dft(const T *t
   dft_any<T, R>(v);
 }
 
-// last stage (Ns = N/R, so k = j): put(j, r, r nb, value) receives row j + r
-// nb.  TOLDS: put writes this column in LDS
+// last stage (Ns = N/R, so k = j): put(j, low, r nb, value) receives row j +
+// r nb; low: r < R/2, for an even radix the rows below N/2 (known at compile
+// time).  TOLDS: put writes this column in LDS
 template <typename T, int MV, bool TOLDS, typename P>
 __device__ __forceinline__ void stage_last(T *lds, const Place &p, int N, int Rs, bool gap, const T *tw, P &&put)
 {
@@ -530,7 +533,7 @@ __device__ __forceinline__ void stage_last(T *lds, const Place &p, int N, int Rs
       if (j < nb) {
         last_dft<T, R>(tw, j, v[u]);
 #pragma unroll
-        for (int r = 0; r < R; r++) put(j, r, r * nb, v[u][r]);
+        for (int r = 0; r < R; r++) put(j, 2 * r < R, r * nb, v[u][r]);
       }
     }
   });
@@ -622,16 +625,20 @@ struct CGeom {
 // threads of a workgroup at most (FP64 butterflies need twice the registers)
 template <typename Real> constexpr int max_threads() { return sizeof(Real) == 4 ? 1024 : 512; }
 
-// strided columns (passes B and D): HIN: only the first N/2 elements are
-// non-zero.  rev: the radices in reversed order (the first radix of a plan
-// is even, the end at which half the elements are missing: the start of pass
-// B, the finish of pass D)
-template <typename Real, bool HIN>
+// which elements of a column a pass reads and keeps, and its direction: FWD
+// (pass B; A of complex charges) reads the first N/2 (the rest are zero) and
+// keeps all, BACK (D; E) transforms backward, in reversed radix order, and
+// keeps the first N/2 (the first radix of a plan is even, the end at which
+// half the elements are missing), WHOLE is any forward transform
+enum { PASS_FWD, PASS_BACK, PASS_WHOLE };
+
+// strided columns (passes B and D)
+template <typename Real, int MODE>
 __global__ __launch_bounds__(max_threads<Real>()) void k_fft_cols(CGeom g, PlanDev pl,
                                                                   const typename Cx<Real>::T *tw,
                                                                   const typename Cx<Real>::T *__restrict__ in,
                                                                   typename Cx<Real>::T *__restrict__ out,
-                                                                  int lgB, int backward)
+                                                                  int lgB)
 {
   using T = typename Cx<Real>::T;
   constexpr int MV = hold<Real, false>();
@@ -645,29 +652,32 @@ __global__ __launch_bounds__(max_threads<Real>()) void k_fft_cols(CGeom g, PlanD
   const int o = valid ? o0 : 0, i = valid ? colg - o0 * g.nInner : 0;
   const T *src = in + ((long)o * g.inOuter + (long)i * g.inInner);
   const T *twl = twiddles_in(lds, column_rows(pl) << lgB, N, tw);
-  const bool rev = backward;
+  constexpr bool rev = MODE == PASS_BACK;
   // an invalid column reads column 0 and is not stored
-  stage_first<T, MV, HIN, false>(lds, p, N, pl.radix[rev ? pl.nst - 1 : 0], [&](int j, int rnb) {
-    T x;
-    if constexpr (HIN) x = (src + (long)j * g.inPos)[(long)rnb * g.inPos];
-    else x = load_or_zero(src, (long)(j + rnb) * g.inPos, j + rnb < g.Lin);
-    return backward ? cconj(x) : x;
+  stage_first<T, MV, MODE == PASS_FWD, false>(lds, p, N, pl.radix[rev ? pl.nst - 1 : 0], [&](int j, int rnb) {
+    if constexpr (MODE == PASS_WHOLE) {
+      return load_or_zero(src, (long)(j + rnb) * g.inPos, j + rnb < g.Lin);
+    } else {
+      const T x = (src + (long)j * g.inPos)[(long)rnb * g.inPos];
+      return rev ? cconj(x) : x;
+    }
   });
   stages_inner<T, MV>(lds, p, pl, rev, twl);
   T *dst = out + ((long)o * g.outOuter + (long)i * g.outInner);
   stage_last<T, MV, false>(lds, p, N, pl.radix[rev ? 0 : pl.nst - 1], pl.nst == 2, twl,
-                       [&](int j, int r, int rnb, T v) {
-    if (valid && j + rnb < g.Lout) (dst + (long)j * g.outPos)[(long)rnb * g.outPos] = backward ? cconj(v) : v;
+                       [&](int j, bool low, int rnb, T v) {
+    const bool keep = MODE == PASS_BACK ? low : MODE == PASS_FWD || j + rnb < g.Lout;
+    if (keep && valid) (dst + (long)j * g.outPos)[(long)rnb * g.outPos] = rev ? cconj(v) : v;
   });
 }
 
 // contiguous rows (passes A and E of complex charges): C rows a workgroup
-template <typename Real, bool HIN>
+template <typename Real, int MODE>
 __global__ __launch_bounds__(max_threads<Real>()) void k_fft_rows(CGeom g, PlanDev pl,
                                                                   const typename Cx<Real>::T *tw,
                                                                   const typename Cx<Real>::T *__restrict__ in,
                                                                   typename Cx<Real>::T *__restrict__ out, int C,
-                                                                  int tpc, int backward)
+                                                                  int tpc)
 {
   using T = typename Cx<Real>::T;
   constexpr int MV = hold<Real, true>();
@@ -681,17 +691,20 @@ __global__ __launch_bounds__(max_threads<Real>()) void k_fft_rows(CGeom g, PlanD
   const T *src = in + (long)i * g.inInner;
   T *dst = out + (long)i * g.outInner;
   const T *twl = twiddles_in(lds, C * column_rows(pl), N, tw);
-  const bool rev = backward;
-  stage_first<T, MV, HIN, false>(lds, p, N, pl.radix[rev ? pl.nst - 1 : 0], [&](int j, int rnb) {
-    T x;
-    if constexpr (HIN) x = (src + j)[rnb];
-    else x = load_or_zero(src, j + rnb, j + rnb < g.Lin);
-    return backward ? cconj(x) : x;
+  constexpr bool rev = MODE == PASS_BACK;
+  stage_first<T, MV, MODE == PASS_FWD, false>(lds, p, N, pl.radix[rev ? pl.nst - 1 : 0], [&](int j, int rnb) {
+    if constexpr (MODE == PASS_WHOLE) {
+      return load_or_zero(src, j + rnb, j + rnb < g.Lin);
+    } else {
+      const T x = (src + j)[rnb];
+      return rev ? cconj(x) : x;
+    }
   });
   stages_inner<T, MV>(lds, p, pl, rev, twl);
   stage_last<T, MV, false>(lds, p, N, pl.radix[rev ? 0 : pl.nst - 1], pl.nst == 2, twl,
-                       [&](int j, int r, int rnb, T v) {
-    if (valid && j + rnb < g.Lout) (dst + j)[rnb] = backward ? cconj(v) : v;
+                       [&](int j, bool low, int rnb, T v) {
+    const bool keep = MODE == PASS_BACK ? low : MODE == PASS_FWD || j + rnb < g.Lout;
+    if (keep && valid) (dst + j)[rnb] = rev ? cconj(v) : v;
   });
 }
 
@@ -718,7 +731,7 @@ __global__ __launch_bounds__(max_threads<Real>()) void k_fft_r2c(int nPairs, int
                               [&](int j, int rnb) { return mk<T>((ra + j)[rnb], (rb + j)[rnb]); });
   stages_inner<T, MV>(lds, p, pl, false, twl);
   stage_last<T, MV, true>(lds, p, N, pl.radix[pl.nst - 1], pl.nst == 2, twl,
-                      [&](int j, int r, int rnb, T v) { (lds + p.at(j))[rnb] = v; });
+                      [&](int j, bool, int rnb, T v) { (lds + p.at(j))[rnb] = v; });
   __syncthreads();
   if (!valid) return;
   const Real h = (Real)0.5;
@@ -734,7 +747,7 @@ __global__ __launch_bounds__(max_threads<Real>()) void k_fft_r2c(int nPairs, int
 
 // pass E: Hermitian half rows -> two real rows (backward transform)
 template <typename Real>
-__global__ __launch_bounds__(max_threads<Real>()) void k_fft_c2r(int Lout, int nPairs, int inRow, int outRow,
+__global__ __launch_bounds__(max_threads<Real>()) void k_fft_c2r(int nPairs, int inRow, int outRow,
                                                                  PlanDev pl, const typename Cx<Real>::T *tw,
                                                                  const typename Cx<Real>::T *__restrict__ in,
                                                                  Real *__restrict__ out, int C, int tpc)
@@ -776,8 +789,8 @@ __global__ __launch_bounds__(max_threads<Real>()) void k_fft_c2r(int Lout, int n
   stage_first<T, MV, false, true>(lds, p, N, pl.radix[pl.nst - 1], [&](int j, int rnb) { return (lds + p.at(j))[rnb]; });
   stages_inner<T, MV>(lds, p, pl, true, twl);
   Real *oa = out + (long)(2 * pr) * outRow, *ob = oa + outRow;
-  stage_last<T, MV, false>(lds, p, N, pl.radix[0], pl.nst == 2, twl, [&](int j, int r, int rnb, T z) {
-    if (valid && j + rnb < Lout) {
+  stage_last<T, MV, false>(lds, p, N, pl.radix[0], pl.nst == 2, twl, [&](int j, bool low, int rnb, T z) {
+    if (low && valid) {
       (oa + j)[rnb] = z.x;  // z: conj of the backward transform
       (ob + j)[rnb] = -z.y;
     }
@@ -861,8 +874,8 @@ __global__ __launch_bounds__(max_threads<Real>()) void k_fft_conv(int nCols, int
     else return mk<T>(gv * x.x, -gv * x.y);
   });
   stages_inner<T, MV>(lds, p, pl, true, twl);
-  stage_last<T, MV, false>(lds, p, N, pl.radix[0], pl.nst == 2, twl, [&](int j, int r, int rnb, T v) {
-    if (valid && j + rnb < N / 2) (col + (long)j * pos)[(long)rnb * pos] = cconj(v);
+  stage_last<T, MV, false>(lds, p, N, pl.radix[0], pl.nst == 2, twl, [&](int j, bool low, int rnb, T v) {
+    if (low && valid) (col + (long)j * pos)[(long)rnb * pos] = cconj(v);
   });
 }
 
@@ -1177,7 +1190,7 @@ __global__ __launch_bounds__(max_threads<double>()) void k_fft_even(int nCols, i
   });
   stages_inner<double2, MV>(lds, p, pl, false, twl);
   stage_last<double2, MV, true>(lds, p, N, pl.radix[pl.nst - 1], pl.nst == 2, twl,
-                            [&](int j, int r, int rnb, double2 v) { (lds + p.at(j))[rnb << p.sh] = v; });
+                            [&](int j, bool, int rnb, double2 v) { (lds + p.at(j))[rnb << p.sh] = v; });
   __syncthreads();
   if (!va) return;
   for (int n = p.tj; n <= h; n += p.tpc) {
@@ -1311,8 +1324,9 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
   c.outPos = (int)g.outPos;
   check_int(g.nCols * std::max<long>(1, g.N), "FFT pass");
   const int L8 = pow8 ? pow8_level(plan) : 0;
-  // half the input: the pruned first stage (forward order: an even radix)
-  const bool half = !backward && 2 * g.Lin == g.N;
+  const int mode = backward ? PASS_BACK : 2 * g.Lin == g.N && g.Lout == g.N ? PASS_FWD : PASS_WHOLE;
+  if (backward && (g.Lin != g.N || 2 * g.Lout != g.N))
+    throw Error{NPME_ERR_ARG, "backward pass: all of a column in, half of it out"};
   const bool half8 = 2 * g.Lin == g.N, full8 = g.Lin == g.N;
   if (!rows && L8 > 0 && (backward ? full8 && 2 * g.Lout == g.N : (half8 || full8) && g.Lout == g.N)) {
     // N = 8^L: the compile-time kernel (4096 / N columns per workgroup)
@@ -1346,22 +1360,24 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
     if (rows)                                                                                  \
       hipLaunchKernelGGL((k_fft_rows<R, H>), grid, dim3(l.T), l.lds, s, c, pd,                 \
                          (const typename Cx<R>::T *)tw, (const typename Cx<R>::T *)in,        \
-                         (typename Cx<R>::T *)out, l.C, l.tpc, (int)backward);                 \
+                         (typename Cx<R>::T *)out, l.C, l.tpc);                                 \
     else                                                                                       \
       hipLaunchKernelGGL((k_fft_cols<R, H>), grid, dim3(l.T), l.lds, s, c, pd,                 \
                          (const typename Cx<R>::T *)tw, (const typename Cx<R>::T *)in,        \
-                         (typename Cx<R>::T *)out, l.lgB, (int)backward);                      \
+                         (typename Cx<R>::T *)out, l.lgB);                                      \
   } while (0)
   const FftLaunch l = rows ? launch_rows(plan, fp64, g.nCols) : launch_cols(plan, fp64, g.nCols);
   const int per = rows ? l.C : 1 << l.lgB;
   const dim3 grid((unsigned)((g.nCols + per - 1) / per));
-  if (fp64) {
-    if (half) NPME_FFTC(double, true);
-    else NPME_FFTC(double, false);
-  } else {
-    if (half) NPME_FFTC(float, true);
-    else NPME_FFTC(float, false);
-  }
+#define NPME_FFTM(R)                                                                           \
+  do {                                                                                         \
+    if (mode == PASS_FWD) NPME_FFTC(R, PASS_FWD);                                              \
+    else if (mode == PASS_BACK) NPME_FFTC(R, PASS_BACK);                                       \
+    else NPME_FFTC(R, PASS_WHOLE);                                                             \
+  } while (0)
+  if (fp64) NPME_FFTM(double);
+  else NPME_FFTM(float);
+#undef NPME_FFTM
 #undef NPME_FFTC
   NPME_HIP_CHECK(hipGetLastError());
 }
@@ -1390,12 +1406,12 @@ void fft_pass_c2r_rows(bool fp64, int N, int Lout, long nRows, long inRowStride,
                        void *out, hipStream_t s)
 {
   check_int(nRows * std::max(inRowStride, outRowStride), "FFT pass");
-  if (plan.N != N) throw Error{NPME_ERR_ARG, "C2R pass: plan of another length"};
+  if (plan.N != N || 2 * Lout != N) throw Error{NPME_ERR_ARG, "C2R pass: rows of N/2 values"};
   const int nPairs = (int)(nRows / 2);
   const FftLaunch l = launch_rows(plan, fp64, nPairs);
   const dim3 grid((unsigned)((nPairs + l.C - 1) / l.C));
 #define NPME_C2R(R)                                                                            \
-  hipLaunchKernelGGL((k_fft_c2r<R>), grid, dim3(l.T), l.lds, s, Lout, nPairs, (int)inRowStride, \
+  hipLaunchKernelGGL((k_fft_c2r<R>), grid, dim3(l.T), l.lds, s, nPairs, (int)inRowStride, \
                      (int)outRowStride, to_dev(plan), (const typename Cx<R>::T *)tw,           \
                      (const typename Cx<R>::T *)in, (R *)out, l.C, l.tpc)
   if (fp64) NPME_C2R(double);
