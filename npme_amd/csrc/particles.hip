@@ -1494,9 +1494,10 @@ void launch_direct_nl(bool fp64, const DirectParams &p, size_t n, const void *sr
 // Positions are in the list walk's frame (the wrapped int32 differences are
 // exact: stencil neighbours are less than 2 clusters apart).  FP32 sums of a
 // group carry into FP64.  The cell-row walk pairs every target of a block of
-// 8 with all charges of the cell rows in reach, 3.7 candidates per pair
-// inside the cutoff at 4 A cells against ~1.6 here: 4M charges in 64 Gaussian
-// blobs (7e10 pairs) 181 -> 81 ms, bound by the ~37 instructions of a pair.
+// 8 with all charges of the cell rows in reach (a stencil of 5^3 cells of 4 A
+// has 3.7 times the volume of the 8 A cutoff sphere): 4M charges in 64 Gaussian
+// blobs (7e10 pairs) 181 -> 81 ms, bound by the VALU: 37 instructions a tested
+// pair at matched order 4 (19 for the difference and the test), 41 at 6, 45 at 8.
 template <typename Real, int KIND, bool FIXP, int MAXD>
 __global__ __launch_bounds__(256) void k_direct_fine(DirectDev p, FineDev g,
                                                      const typename V4t<Real>::T *__restrict__ src,

@@ -27,6 +27,7 @@ def test_refpairs_match_oracle(oracle, nNeigh, nClust, packed):
     h = N.NPME_Interface_SetUpRealKernel(k, len(q), coord)
     assert h is not None, N.npme_last_error()
     V = h.calcv(q)
+    assert np.array_equal(V, h.calcv(q)) and np.array_equal(V, h.calcv(q))  # graph replays
     ko = oracle.kernel_erf(6.0, oracle.rdir2beta(6.0, 1e-6))
     m = oracle.compare_v(oracle.calcv_laplace_orig(ko, (64, 64, 64), 6, coord, q, nNeigh=nNeigh,
                                                    nCellClust1D=nClust), V)
