@@ -1162,17 +1162,26 @@ __device__ __forceinline__ void pair_sr(const DirectDev &p, Real rx, Real ry, Re
     part[7] += rz * gi;
   } else if constexpr (KIND == KIND_RALPHA_HALF) {
     // FP32: r^alpha = r^raPow sqrt(r)^raHalf by hardware roots and products
-    // in two-part arithmetic, rounded once (the branches are uniform).  r^0.5
-    // at 200k charges: 121 -> 49 us against pow and a division
-    Two r, ri, fe = {1.0f, 0.0f};
-    two_root({r2, 0.0f}, r, ri);
-    if (p.raHalf) {
-      Two hi;
-      two_root(r, fe, hi);
+    // in two-part arithmetic, rounded once (those branches are uniform).  r^0.5
+    // at 200k charges: 121 -> 49 us against pow and a division.  Pairs closer
+    // than 1e-6, coincident charges among them, take pow and the division: 0,
+    // infinities and overflow have no low part (0 inf and inf - inf there made
+    // V of coincident charges NaN), and from 1e-6 on r^-5 = 1e30 is in range
+    Two fe = {1.0f, 0.0f}, fd;
+    if (r2 < 1.0e-12f) {  // rare
+      fe.hi = pow(r2, (Real)(0.5 * p.alpha));
+      fd = {fe.hi / r2, 0.0f};
+    } else {
+      Two r, ri;
+      two_root({r2, 0.0f}, r, ri);
+      if (p.raHalf) {
+        Two hi;
+        two_root(r, fe, hi);
+      }
+      const Two m = p.raPow >= 0 ? r : ri;
+      for (int k = abs(p.raPow); k > 0; k--) fe = two_mul(fe, m);
+      fd = two_mul(fe, two_mul(ri, ri));
     }
-    const Two m = p.raPow >= 0 ? r : ri;
-    for (int k = abs(p.raPow); k > 0; k--) fe = two_mul(fe, m);
-    const Two fd = two_mul(fe, two_mul(ri, ri));
     const Real f0 = (fe.hi - horner_top<Real, MAXD>(topA, coef_a<Real>(p), r2)) + fe.lo;
     const Real f1 = (Real)p.alpha * (fd.hi + fd.lo) - horner_top<Real, MAXD>(topB, coef_b<Real>(p), r2);
     const Real fq = f1 * qr;

@@ -65,3 +65,37 @@ def test_helmholtz_pairs(oracle, k0, lists):
     k0 = complex(k0)
     _run(oracle, "Helmholtz", oracle.kernel(oracle.HELMHOLTZ, 6, 6.0, k0=k0), coord, q, k0_r=k0.real,
          k0_i=k0.imag, neighborList=lists)
+
+
+@pytest.mark.parametrize("side", [20.0, 8.0])
+@pytest.mark.parametrize("alpha", [0.5, 1.0, 3.0, -0.5, -2.0, 0.3])
+def test_ralpha_coincident_charges(alpha, side):
+    """Two charges at one place, in the cell rows and in dense cells: V is
+    what the FP64 walk gives (r^alpha is 0 or infinite there, never NaN; 1e-5,
+    ten times the mixed form's bound for a set), and the other charges' V and
+    gradients are those of the list walk, which has the same grid part and the
+    same pair terms summed in another order."""
+    import npme_amd as N
+    print("case coincident charges", alpha, side, flush=True)
+    coord, q = uniform_box(1500, side)
+    coord[11] = coord[10]
+    V = {}
+    for prec, lists in (("fp64", "off"), ("mixed", "off"), ("mixed", "on")):
+        k = N.NPME_KeywordInput(calcType="pme", funcType="Ralpha", EwaldSplit="DerivMatch", Rdir=6.0, BnOrder=6,
+                                tol=1e-6, precision=prec, N1=64, N2=64, N3=64, n1=16, n2=16, n3=16, nDeriv=6,
+                                alpha=alpha, neighborList=lists)
+        assert N.NPME_AddMissingKeywords(k, len(q), coord, chargeReal=q), N.npme_last_error()
+        h = N.NPME_Interface_SetUpRealKernel(k, len(q), coord)
+        assert h is not None, N.npme_last_error()
+        assert ("neighbour list" if lists == "on" else "dense cells" if side == 8.0 else "cell rows") in h.Print()
+        V[prec, lists] = h.calcv(q)
+    at = np.array([10, 11])
+    far = np.setdiff1d(np.arange(len(q)), at)
+    a, b, c = V["mixed", "off"], V["fp64", "off"], V["mixed", "on"]
+    rms = np.sqrt(np.mean(c[far, 0] ** 2))
+    if alpha > 0:
+        assert np.isfinite(a[at, 0]).all() and np.abs(a[at, 0] - b[at, 0]).max() < 1e-5 * rms, (a[at, 0], b[at, 0])
+    else:
+        assert np.array_equal(a[at, 0], b[at, 0]) and np.isinf(a[at, 0]).all(), (a[at, 0], b[at, 0])
+    assert np.sqrt(np.mean((a[far, 0] - c[far, 0]) ** 2)) < 1e-6 * rms
+    assert np.sqrt(np.mean((a[far, 1:] - c[far, 1:]) ** 2)) < 5e-6 * np.sqrt(np.mean(c[far, 1:] ** 2))
