@@ -502,7 +502,8 @@ int npme_print(const npme_handle *h, char *buf, size_t buflen)
   if (H.trans)
     os << "  direct sum: none (box pair on the translated kernel grid)\n";
   else if (kind_ref_pairs(H.ker.kind))
-    os << "  direct sum: the reference's interacting cell pairs, every point pair (FP64)\n";
+    os << "  direct sum: the reference's interacting cell pairs, every point pair (FP64)"
+       << (H.nRefBlocks ? ", " + std::to_string(H.nRefBlocks) + " wavefronts" : std::string()) << "\n";
   else if (H.useNlist)
     os << "  direct sum: neighbour list, " << H.nlistEntries << " entries\n";
   else if (H.useFine)

@@ -349,6 +349,8 @@ struct Handle {
   double *d_coordS = nullptr;    // [n][3] FP64 input coordinates, input order (exact sums)
   double4 *d_xs = nullptr;       // [n] FP64 coordinates in sorted order (pair search)
   unsigned *d_cellFlags = nullptr;  // LaplaceOrig: interacting (cell, stencil offset) bits
+  int2 *d_refBlk = nullptr;      // and its wavefronts' (cell, first target), kRefTargets targets each
+  int nRefBlocks = 0;            // 0: a thread per target
   FFTPlan1D plan[3];
   AxisTables axis[3];            // host tables of the grid sizes (grid_setup)
   size_t deviceBytes = 0;
@@ -425,6 +427,8 @@ void geometry_charges_device(const GeoParams &g, bool fp64, size_t n, const doub
                              void *d_frac, DevBuf &tileStart, DevBuf &tileList, DevBuf &itileStart,
                              DevBuf &itileList, size_t &nTileEntries, bool listSentinel,
                              bool &sentinelPlaced, hipStream_t s);
+// targets of one cell that a wavefront of k_direct_refpairs_cell takes
+constexpr int kRefTargets = 8;
 // fine order of densely packed charges (k_direct_fine): blocks of 64 charges
 // of one cell in kFineSub groups of kFineGroup
 constexpr int kFineGroup = 16, kFineSub = 64 / kFineGroup;
@@ -550,8 +554,17 @@ double handle_count_pairs(Handle &h);
 int refpair_words(int nNeigh);
 void launch_cellpair_contact(const DirectParams &pp, const int *cellStart, const double4 *xs,
                              unsigned *flags, hipStream_t s);
+// blk: nBlocks (cell, first target) items of kRefTargets targets, none for
+// stencils wider than refpair_cells admits (a thread per target)
+bool refpair_cells(int nNeigh);
+// the items, in any order, and their number (count: zeroed); a cell of c
+// charges has ceil(c / kRefTargets), so n / kRefTargets and one for each
+// occupied cell bound them
+inline size_t refpair_max_blocks(size_t n, size_t ncell) { return n / kRefTargets + std::min(n, ncell); }
+void launch_refpair_blocks(const DirectParams &pp, size_t n, const int4 *cell, const int *cellStart, int *count,
+                           int2 *blk, hipStream_t s);
 void launch_direct_refpairs(const DirectParams &pp, size_t n, const int4 *cell, const int *cellStart,
-                            const double4 *xs, const int *perm, const double *q,
+                            const int2 *blk, int nBlocks, const double4 *xs, const int *perm, const double *q,
                             const unsigned *flags, double *Vdir, hipStream_t s);
 // kernels whose direct sum takes the reference's pair set (no cutoff):
 // LaplaceOrig's erfc and the user-defined short-range parts

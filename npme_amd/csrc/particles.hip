@@ -1819,17 +1819,23 @@ __global__ __launch_bounds__(256) void k_cellpair_contact(DirectDev p, long ncel
   if (on) atomicOr(&flags[c * W + (o >> 5)], 1u << (o & 31));
 }
 
-// Stencils up to nNeigh = NLW_NN: a wavefront per cell.  The targets of a
-// cell share its flagged cells, so the wavefront enumerates their charges once
-// per batch of targets (counts scanned into LDS, each lane finding its charge
+// Stencils up to nNeigh = NLW_NN: a wavefront per kRefTargets targets of one
+// cell (blk: cell and first target; a sparse cell is one wavefront's, the
+// targets of a crowded one spread over the chip).  The targets of a cell share
+// its flagged cells, so the wavefront enumerates their charges once per batch
+// of targets (counts scanned into LDS, each lane finding its charge
 // by a binary search), one charge per lane, 64 at a time, and evaluates them
 // against each target of the batch in turn; the lanes' FP64 sums are added
 // at the batch's end.  What bounds it is FP64 arithmetic (erfc and exp, ~200
 // instructions a pair): a thread per target, which chased cell, charge index
 // and charge through dependent loads with 1.5 wavefronts a SIMD, took 560 us
-// for 100k charges (~3e7 pairs), this 199 us.
+// for 100k charges (~3e7 pairs), this 192 us.  A whole cell to a wavefront is
+// as good there (2.7 charges a cell) and worse the fuller the cells: 2,500
+// charges in one cell 42 ms, 0.18 ms shared out (a thread per target: 3.3),
+// 20,000 in a blob 146 ms and 2.5 ms (13.5).
 template <int KIND>
-__global__ __launch_bounds__(256) void k_direct_refpairs_cell(DirectDev p, long ncell, int W,
+__global__ __launch_bounds__(256) void k_direct_refpairs_cell(DirectDev p, int nBlocks, int W,
+                                                              const int2 *__restrict__ blk,
                                                               const int2 *__restrict__ cellSE,
                                                               const double4 *__restrict__ xs,
                                                               const int *__restrict__ perm,
@@ -1842,10 +1848,12 @@ __global__ __launch_bounds__(256) void k_direct_refpairs_cell(DirectDev p, long 
   __shared__ int shStart[4][NLW_MAXC];
   __shared__ int shPre[4][NLW_MAXC];
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  const long c = (long)blockIdx.x * 4 + w;
-  if (c >= ncell) return;  // uniform per wavefront; no workgroup barrier below
+  const int b = blockIdx.x * 4 + w;
+  if (b >= nBlocks) return;  // uniform per wavefront; no workgroup barrier below
+  const int2 item = blk[b];
+  const long c = item.x;
   const int2 home = cellSE[c];
-  if (home.y == 0) return;
+  const int tEnd = min(home.y, item.y + kRefTargets);
   const int hz = (int)(c % p.nb2), hy = (int)((c / p.nb2) % p.nb1), hx = (int)(c / ((long)p.nb1 * p.nb2));
   const int nN = p.nNeigh, S = 2 * nN + 1, M = S * S * S;
   int T = 0;
@@ -1871,8 +1879,8 @@ __global__ __launch_bounds__(256) void k_direct_refpairs_cell(DirectDev p, long 
     T += __shfl(inc, 63);
   }
   wave_lds_order();
-  for (int tb = 0; tb < home.y; tb += TB) {
-    const int mt = min(TB, home.y - tb), s0 = home.x + tb;
+  for (int tb = item.y; tb < tEnd; tb += TB) {
+    const int mt = min(TB, tEnd - tb), s0 = home.x + tb;
     double part[TB][8];
 #pragma unroll
     for (int i = 0; i < TB; i++)
@@ -1985,27 +1993,49 @@ void launch_cellpair_contact(const DirectParams &pp, const int *cellStart, const
   // the reference's test: Rdir recomputed as nNeigh cell edges, squared
   // distance below 1.0001 Rdir^2 (src/PartitionBox.cpp:767-787, :841-842)
   const double cs = pp.Rdir / pp.nNeigh, Rr = pp.nNeigh * cs, R2 = Rr * Rr * 1.0001;
-  NPME_HIP_CHECK(hipMemsetAsync(flags, 0, (size_t)ncell * W * sizeof(unsigned), s));
+  // and the work item count behind the flags
+  NPME_HIP_CHECK(hipMemsetAsync(flags, 0, ((size_t)ncell * W + 1) * sizeof(unsigned), s));
   const long tot = ncell * S * S * S;
   hipLaunchKernelGGL(k_cellpair_contact, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, d, ncell, W,
                      R2, (const int2 *)cellStart, xs, flags);
   NPME_HIP_CHECK(hipGetLastError());
 }
 
+// a thread per sorted charge: every kRefTargets-th of a cell starts an item
+__global__ __launch_bounds__(256) void k_refpair_blocks(size_t n, int nb1, int nb2, const int4 *__restrict__ cell,
+                                                        const int2 *__restrict__ cellSE, int *__restrict__ count,
+                                                        int2 *__restrict__ blk)
+{
+  const size_t s = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const int4 g = cell[s];
+  const long c = ((long)g.x * nb1 + g.y) * nb2 + g.z;
+  const int r = (int)s - cellSE[c].x;
+  if (r % kRefTargets == 0) blk[atomicAdd(count, 1)] = make_int2((int)c, r);
+}
+void launch_refpair_blocks(const DirectParams &pp, size_t n, const int4 *cell, const int *cellStart, int *count,
+                           int2 *blk, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_refpair_blocks, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, pp.nb[1], pp.nb[2],
+                     cell, (const int2 *)cellStart, count, blk);
+  NPME_HIP_CHECK(hipGetLastError());
+}
+
+bool refpair_cells(int nNeigh) { return nNeigh <= NLW_NN; }
+
 void launch_direct_refpairs(const DirectParams &pp, size_t n, const int4 *cell, const int *cellStart,
-                            const double4 *xs, const int *perm, const double *q,
+                            const int2 *blk, int nBlocks, const double4 *xs, const int *perm, const double *q,
                             const unsigned *flags, double *Vdir, hipStream_t s)
 {
   const DirectDev d = refpair_dev(pp);
   const int W = refpair_words(pp.nNeigh);
-  const long ncell = (long)pp.nb[0] * pp.nb[1] * pp.nb[2];
-  const bool cells = pp.nNeigh <= NLW_NN;
+  const bool cells = refpair_cells(pp.nNeigh);
   const int2 *cse = (const int2 *)cellStart;
 #define NPME_REFPAIRS(K)                                                                         \
   do {                                                                                           \
     if (cells)                                                                                   \
-      hipLaunchKernelGGL(k_direct_refpairs_cell<K>, dim3((unsigned)((ncell + 3) / 4)), dim3(256), 0, s, d, \
-                         ncell, W, cse, xs, perm, q, flags, Vdir);                               \
+      hipLaunchKernelGGL(k_direct_refpairs_cell<K>, dim3((unsigned)((nBlocks + 3) / 4)), dim3(256), 0, s, d, \
+                         nBlocks, W, blk, cse, xs, perm, q, flags, Vdir);                        \
     else                                                                                         \
       hipLaunchKernelGGL(k_direct_refpairs<K>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d, n, W, \
                          cell, cse, xs, perm, q, flags, Vdir);                                   \

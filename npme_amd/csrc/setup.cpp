@@ -64,7 +64,7 @@ void handle_free_device(Handle &h, bool keepG)
                   h.d_sliceStart, h.d_sliceLen, h.d_qi, h.d_cell, h.d_cellStart, h.d_ms, h.d_frac,
                   h.d_tileStart, h.d_tileList, h.d_grid, h.d_buf1, h.d_buf2,
                   h.d_tables, h.d_Vdir, h.d_V, h.d_qin, h.d_coordS, h.d_xs,
-                  h.d_qs, h.d_qsi, h.d_utab, h.d_cellFlags, h.d_fineOrder, h.d_finePerm, h.d_fineStart,
+                  h.d_qs, h.d_qsi, h.d_utab, h.d_cellFlags, h.d_refBlk, h.d_fineOrder, h.d_finePerm, h.d_fineStart,
                   h.d_fineBlk, h.d_fineBox};
   // queued work of this handle may still read its buffers
   if (h.stream) (void)hipStreamSynchronize(h.stream);
@@ -98,6 +98,8 @@ void handle_free_device(Handle &h, bool keepG)
   h.d_xs = nullptr;
   h.d_utab = nullptr;
   h.d_cellFlags = nullptr;
+  h.d_refBlk = nullptr;
+  h.nRefBlocks = 0;
   h.d_fineOrder = h.d_finePerm = h.d_fineStart = nullptr;
   h.d_fineBlk = nullptr;
   h.d_fineBox = nullptr;
@@ -1283,8 +1285,17 @@ void handle_setup(Handle &h, const Keywords &kw, size_t n, const double *coord)
   }
   if (kind_ref_pairs(h.ker.kind)) {
     const size_t ncell = (size_t)h.nb[0] * h.nb[1] * h.nb[2];
-    h.d_cellFlags = dalloc<unsigned>(h, ncell * refpair_words((int)h.nNeigh));
-    launch_cellpair_contact(direct_params(h), h.d_cellStart, h.d_xs, h.d_cellFlags, h.stream);
+    // the flags, and the number of work items behind them (cleared with them)
+    const size_t words = ncell * refpair_words((int)h.nNeigh);
+    h.d_cellFlags = dalloc<unsigned>(h, words + 1);
+    const DirectParams dp = direct_params(h);
+    launch_cellpair_contact(dp, h.d_cellStart, h.d_xs, h.d_cellFlags, h.stream);
+    if (refpair_cells((int)h.nNeigh)) {
+      int *count = reinterpret_cast<int *>(h.d_cellFlags + words);
+      h.d_refBlk = dalloc<int2>(h, refpair_max_blocks(h.n, ncell));
+      launch_refpair_blocks(dp, h.n, h.d_cell, h.d_cellStart, count, h.d_refBlk, h.stream);
+      NPME_HIP_CHECK(hipMemcpyAsync(&h.nRefBlocks, count, sizeof(int), hipMemcpyDeviceToHost, h.stream));
+    }
     NPME_HIP_CHECK(hipStreamSynchronize(h.stream));
   }
   grid_setup(h);
@@ -1407,8 +1418,8 @@ static void calcv_launches(Handle &h, const double *d_q, double *d_Vout, bool sp
   };
   auto direct = [&](hipStream_t ds) {
     if (refPairs)
-      launch_direct_refpairs(dp, h.n, h.d_cell, h.d_cellStart, h.d_xs, h.d_perm, d_q, h.d_cellFlags,
-                             h.d_Vdir, ds);
+      launch_direct_refpairs(dp, h.n, h.d_cell, h.d_cellStart, h.d_refBlk, h.nRefBlocks, h.d_xs, h.d_perm, d_q,
+                             h.d_cellFlags, h.d_Vdir, ds);
     else if (h.useFine)
       launch_direct_fine(f64, dp,
                          FineDev{h.nFineBlocks, h.d_fineBlk, (const int2 *)h.d_cellStart, h.d_fineStart, h.d_fineBox,
