@@ -1244,7 +1244,7 @@ void handle_setup(Handle &h, const Keywords &kw, size_t n, const double *coord)
     };
     // grids with few tiles take smaller ones, down to edge 4, until every CU
     // has one: a launch of 27 workgroups is as long as one of them (96^3
-    // grid, 22k charges: 27 tiles of edge 16 30 us, 216 of edge 8 13 us)
+    // grid, 22k charges: 27 tiles of edge 16 30 us, 216 of edge 8 10 us)
     const int edges[] = {16, 12, 8, 6, 4, 2, 1};
     for (int e : edges) {
       h.TI = e;

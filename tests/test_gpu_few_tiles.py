@@ -45,3 +45,34 @@ def test_few_tiles_match_oracle(oracle, n, grid, Bn, packed, kind, prec):
     print(m["relV"], m["reldV"])
     bound = (1e-11, 1e-11) if prec == "fp64" else (1e-6, 1e-5)
     assert m["relV"] < bound[0] and m["reldV"] < bound[1], m
+
+
+def _interp_us(n, packed):
+    """Interpolation stage of a set of n charges on a 64^3 grid: the fastest of
+    40 calls (device time between events)."""
+    import npme_amd as N
+    coord, q = uniform_box(n, 32.0)
+    if packed:
+        coord[2:] = 16.0 + 0.06 * (coord[2:] - 16.0)
+        coord[0], coord[1] = 0.0, 32.0
+    k = N.NPME_KeywordInput(calcType="pme", funcType="Laplace", EwaldSplit="DerivMatch", Rdir=5.0, BnOrder=6, tol=1e-6,
+                            precision="mixed", N1=64, N2=64, N3=64, n1=16, n2=16, n3=16, nDeriv=6)
+    assert N.NPME_AddMissingKeywords(k, n, coord, chargeReal=q), N.npme_last_error()
+    h = N.NPME_Interface_SetUpRealKernel(k, n, coord)
+    assert h is not None, N.npme_last_error()
+    h.set_profiling(True)
+    times = []
+    for _ in range(40):
+        h.calcv(q)
+        times.append(h.stage_times()[-1])
+    return 1e3 * min(times)
+
+
+def test_crowded_interpolation_tile():
+    """6,000 charges that fall into a few tiles of edge 4: their tile must
+    have a whole block of wavefronts.  About 8 times the time of the same
+    number spread out, and 24 times with one wavefront a tile: bound 14."""
+    print("case crowded tile", flush=True)
+    spread, packed = _interp_us(6000, False), _interp_us(6000, True)
+    print(spread, packed)
+    assert packed < 14 * spread
