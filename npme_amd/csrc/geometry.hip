@@ -334,17 +334,27 @@ __global__ __launch_bounds__(256) void k_tile_scan(size_t n, TileGrid g, long nw
     }
     unsigned long long todo = __ballot(hit);
     while (todo) {  // uniform
-      const int l = __ffsll((unsigned long long)todo) - 1;
-      todo &= todo - 1;
-      const size_t s = (size_t)(c0 + l) * 64 + lane;
-      bool in = false;
-      if (s < n) {
-        const int4 u = ms[s];
-        in = u.x >= lo[0] && u.x <= hi[0] && u.y >= lo[1] && u.y <= hi[1] && u.z >= lo[2] && u.z <= hi[2];
+      // up to four chunks at a time, their loads in flight together
+      size_t s[4];
+      int4 u[4];
+      bool have[4];
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        have[v] = todo != 0;
+        const int l = have[v] ? __ffsll((unsigned long long)todo) - 1 : 0;
+        todo &= todo - 1;  // 0 stays 0
+        s[v] = (size_t)(c0 + l) * 64 + lane;
+        have[v] = have[v] && s[v] < n;
+        u[v] = ms[have[v] ? s[v] : 0];
       }
-      const unsigned long long m = __ballot(in);
-      if (FILL && in) out[k + __popcll(m & ((1ull << lane) - 1))] = (int)s;
-      k += __popcll(m);
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const bool in = have[v] && u[v].x >= lo[0] && u[v].x <= hi[0] && u[v].y >= lo[1] && u[v].y <= hi[1] &&
+                        u[v].z >= lo[2] && u[v].z <= hi[2];
+        const unsigned long long m = __ballot(in);
+        if (FILL && in) out[k + __popcll(m & ((1ull << lane) - 1))] = (int)s[v];
+        k += __popcll(m);
+      }
     }
   }
   if (!FILL && lane == 0) out[w] = k;
@@ -597,7 +607,10 @@ struct TileScan {
       nt *= ntd[d];
     }
     g.width = width;
-    g.Q = nt < 512 ? 8 : nt < 4096 ? 2 : 1;  // wavefronts for every SIMD
+    // parts of a tile: wavefronts for the whole chip (16 a SIMD) of at least 8
+    // chunks each, and of at most 256, since all charges may be in one tile
+    const long nch = (long)((n + 63) / 64);
+    g.Q = (int)std::max({1L, std::min(16384 / nt, (nch + 7) / 8), (nch + 255) / 256});
     nw = nt * g.Q;
     cnt.reset((nw + 1) * sizeof(int));
     part.reset((nw + 1) * sizeof(int));
