@@ -38,7 +38,7 @@ __device__ __forceinline__ bool d_coord2cell(double x, double cs, unsigned long 
 }
 
 __global__ __launch_bounds__(256) void k_cell_keys(size_t n, const double *__restrict__ coord,
-                                                   GeoParams g, unsigned *__restrict__ key,
+                                                   GeoParams g, int bits, unsigned *__restrict__ key,
                                                    int *__restrict__ slot, int *__restrict__ count,
                                                    int4 *__restrict__ gcell, int *__restrict__ err)
 {
@@ -61,7 +61,20 @@ __global__ __launch_bounds__(256) void k_cell_keys(size_t n, const double *__res
   const unsigned long tA = (a[0] * g.nA[1] + a[1]) * g.nA[2] + a[2];
   const unsigned k = (unsigned)(tA * Nc + (b[0] * g.nP + b[1]) * g.nP + b[2]);
   key[i] = k;
-  slot[i] = atomicAdd(&count[k], 1);
+  // one atomic for the charges of a wavefront that share a cell: atomics on
+  // one address are served ~7 ns apart, so 22k charges in a ball of one cell
+  // took 146 us with an atomic each
+  const int lane = threadIdx.x & 63;
+  unsigned long long m = __ballot(1);  // lanes of the same cell
+  for (int b2 = 0; b2 < bits; b2++) {  // uniform
+    const bool one = (k >> b2) & 1u;
+    const unsigned long long ones = __ballot(one);
+    m &= one ? ones : ~ones;
+  }
+  const int lead = __ffsll(m) - 1, before = __popcll(m & ((1ull << lane) - 1));
+  int first = 0;
+  if (lane == lead) first = atomicAdd(&count[k], __popcll(m));
+  slot[i] = __shfl(first, lead) + before;
   gcell[i] = make_int4((int)(a[0] * g.nP + b[0]), (int)(a[1] * g.nP + b[1]),
                        (int)(a[2] * g.nP + b[2]), 0);
 }
@@ -99,8 +112,14 @@ __global__ __launch_bounds__(256) void k_cell_place(size_t n, const unsigned *__
 // rank of value v among the entries [b, e) of its bucket (distinct values)
 __device__ __forceinline__ int bucket_rank(const int *__restrict__ tmp, int b, int e, int v)
 {
-  int r = 0;
-  for (int f = b; f < e; f++) r += tmp[f] < v;
+  int r = 0, f = b;
+  for (; f < e && (f & 3); f++) r += tmp[f] < v;
+#pragma unroll 8
+  for (; f + 4 <= e; f += 4) {
+    const int4 t = *reinterpret_cast<const int4 *>(tmp + f);
+    r += (t.x < v) + (t.y < v) + (t.z < v) + (t.w < v);
+  }
+  for (; f < e; f++) r += tmp[f] < v;
   return r;
 }
 
@@ -120,8 +139,8 @@ __global__ __launch_bounds__(256) void k_cell_rank(size_t n, const int *__restri
   const unsigned k = key[i];
   const int b = start[k], e = start[k + 1];
   size_t o = p;
-  if (e - b > kRankMax) atomicOr(err, GEO_LONG_BUCKET);
-  else o = (size_t)b + bucket_rank(tmp, b, e, i);
+  if (e - b <= kRankMax) o = (size_t)b + bucket_rank(tmp, b, e, i);
+  else if (p == (size_t)b) atomicOr(err, GEO_LONG_BUCKET);  // one charge of the cell
   perm[o] = i;
   cellOf[o] = gcell[i];
   xs[o] = make_double4(coord[3 * (size_t)i], coord[3 * (size_t)i + 1], coord[3 * (size_t)i + 2], 0.0);
@@ -549,8 +568,8 @@ void geometry_cells_device(const GeoParams &g, size_t n, const double *d_coord, 
       slot(n * sizeof(int)), tmp(n * sizeof(int)), gcell(n * sizeof(int4));
   int *count = (int *)cnt.p, *err = count + ncell + 1;
   zero_words((size_t)ncell + 2, count, s);
-  hipLaunchKernelGGL(k_cell_keys, grid_for(n), dim3(256), 0, s, n, d_coord, g, (unsigned *)key.p,
-                     (int *)slot.p, count, (int4 *)gcell.p, err);
+  hipLaunchKernelGGL(k_cell_keys, grid_for(n), dim3(256), 0, s, n, d_coord, g,
+                     key_bits((unsigned long)ncell), (unsigned *)key.p, (int *)slot.p, count, (int4 *)gcell.p, err);
   NPME_HIP_CHECK(hipGetLastError());
   // a charge outside the box gets key 0 and cell 0, so the sort and the
   // ranges stay in bounds; the error is raised after the phase
@@ -965,13 +984,18 @@ __global__ __launch_bounds__(256) void k_fine_count(long ncell, const int2 *__re
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c <= ncell) count[c] = c < ncell ? (cellSE[c].y + 63) / 64 : 0;
 }
-__global__ __launch_bounds__(256) void k_fine_blocks(long ncell, const int2 *__restrict__ cellSE,
+// a thread per sorted charge, since a cell may hold any number of them (with a
+// thread per cell, 1M charges in a ball of 27 cells took 328 us)
+__global__ __launch_bounds__(256) void k_fine_blocks(size_t n, int nb1, int nb2, const int4 *__restrict__ cellOf,
+                                                     const int2 *__restrict__ cellSE,
                                                      const int *__restrict__ blkStart, int2 *__restrict__ blk)
 {
-  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncell) return;
-  const int nb = (cellSE[c].y + 63) / 64;
-  for (int k = 0; k < nb; k++) blk[blkStart[c] + k] = make_int2((int)c, 64 * k);
+  const size_t s = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const int4 g = cellOf[s];
+  const long c = ((long)g.x * nb1 + g.y) * nb2 + g.z;
+  const int r = (int)s - cellSE[c].x;
+  if (r % 64 == 0) blk[blkStart[c] + r / 64] = make_int2((int)c, r);
 }
 // sort key: the first charge of the cell (cells keep their order), then the
 // Morton index of the position in the cell, 16 steps an axis
@@ -1056,10 +1080,10 @@ void fine_order_device(const GeoParams &g, size_t n, int nBlocks, const double4 
                        const int *d_cellSE, const int *d_perm, const int *d_blkStart, int *d_order, int *d_permF,
                        int2 *d_blk, float4 *d_box, hipStream_t s)
 {
-  const long ncell = (long)g.nb[0] * g.nb[1] * g.nb[2];
   const int2 *cse = (const int2 *)d_cellSE;
   DevBuf key(n * sizeof(unsigned long)), skey(n * sizeof(unsigned long)), idx(n * sizeof(int));
-  hipLaunchKernelGGL(k_fine_blocks, grid_for(ncell), dim3(256), 0, s, ncell, cse, d_blkStart, d_blk);
+  hipLaunchKernelGGL(k_fine_blocks, grid_for(n), dim3(256), 0, s, n, g.nb[1], g.nb[2], d_cellOf, cse, d_blkStart,
+                     d_blk);
   hipLaunchKernelGGL(k_fine_keys, grid_for(n), dim3(256), 0, s, n, g, d_xs, d_cellOf, cse,
                      (unsigned long *)key.p, (int *)idx.p);
   NPME_HIP_CHECK(hipGetLastError());

@@ -73,3 +73,17 @@ def test_few_tiles_cost():
     few, many = _reset_ms(coord, q, 40), _reset_ms(coord, q, 128)
     print(few, many)
     assert few < 1.15 * many
+
+
+def test_crowded_cells_cost():
+    """200,000 charges in a few dozen cells against the same number spread
+    over the box: counting, ranking and block lists do not serialise on a
+    crowded cell (3 times the time when they did)."""
+    print("case crowded cells cost", flush=True)
+    coord, q = uniform_box(200000, 60.0)
+    spread = _reset_ms(coord, q, 96)
+    coord[2:] = 31.0 + 0.03 * (coord[2:] - 30.0)
+    coord[0], coord[1] = 0.0, 60.0
+    crowded = _reset_ms(coord, q, 96)
+    print(crowded, spread)
+    assert crowded < 1.5 * spread
