@@ -44,7 +44,7 @@ struct DirectDev {
   double fxInvD;     // fxInv in FP64 (scale of the list walk's gradient sums)
   float fxClose2u;   // list walk: squared distance in fixed-point units below which
                      // a pair adds the residuals (2^48: pairs closer than 2^24 units)
-  float k0q[2];      // k0r 2 / pi split in two FP32 parts (phase in quarter turns)
+  double k0q;        // k0r 2 / pi (phase in quarter turns)
   int raPow, raHalf; // KIND_RALPHA_HALF: alpha = raPow + raHalf / 2
   const void *utab;  // user kernels: short-range table in the working precision
   int utS;           // pieces per octave of the table
@@ -417,9 +417,7 @@ static DirectDev direct_dev(const DirectParams &p)
   d.eshift = p.nlEshift;
   d.fxInvD = p.fxInv;
   d.fxClose2u = 281474976710656.0f;  // 2^48
-  const double kq = p.k0r * 0.63661977236758134308;
-  d.k0q[0] = (float)kq;
-  d.k0q[1] = (float)(kq - (double)d.k0q[0]);
+  d.k0q = p.k0r * 0.63661977236758134308;
   d.raPow = (int)std::floor(p.alpha);
   d.raHalf = 2.0 * p.alpha != 2.0 * d.raPow;
   return d;
@@ -1075,20 +1073,19 @@ __device__ __forceinline__ void two_root(Two x, Two &rt, Two &inv)
   inv.lo = y * fmaf(-rt.lo, y, fmaf(-rt.hi, y, 1.0f));
 }
 
-// cos and sin of pi/2 (khi + klo) r in FP32.  The phase in quarter turns is
-// r khi exactly as a sum of two FP32 numbers (fma), so removing the nearest
-// integer leaves the fraction t in [-1/2, 1/2] with an error of half an ulp
-// of 1/2 whatever the phase, as good as a reduction in FP64; sin and cos of
-// pi/2 t are minimax polynomials in t^2 (relative errors 3.8e-9 and 6.4e-11,
-// fitted by Lawson's iteration; FP32 evaluation 4.2e-8 and 5.7e-8 absolute).
-// ~25 instructions, against ~95 for the FP64 reduction and the library's
-// sincosf with its own.
-__device__ __forceinline__ void phase_sincos(float r, float khi, float klo, float &sn, float &cn)
+// cos and sin of k0r r in FP32 with the phase reduced in FP64, kq = 2 k0r / pi:
+// adding 1.5 2^52 leaves the phase in whole quarter turns in the low bits of
+// the sum (|phase| < 2^31), and the remainder t in [-1/2, 1/2] is rounded once;
+// sin and cos of pi/2 t are minimax polynomials in t^2 (relative errors 3.8e-9
+// and 6.4e-11, fitted by Lawson's iteration; FP32 evaluation 4.2e-8 and 5.7e-8
+// absolute).  The library's sincosf, with its own reduction behind the FP64
+// one, took ~95 instructions, this 20.
+__device__ __forceinline__ void phase_sincos(float r, double kq, float &sn, float &cn)
 {
 #pragma clang fp contract(off)
-  const float pq = r * khi;
-  const float n = __builtin_rintf(pq);
-  const float t = (pq - n) + fmaf(r, klo, fmaf(r, khi, -pq));
+  const double big = 6755399441055744.0;
+  const double rd = (double)r, sum = fma(rd, kq, big);
+  const float t = (float)fma(rd, kq, big - sum);
   const float s = t * t;
   float a = fmaf(s, -0.0046048265110679235f, 0.07968141056178463f);
   a = fmaf(s, a, -0.6459636300573146f);
@@ -1098,7 +1095,7 @@ __device__ __forceinline__ void phase_sincos(float r, float khi, float klo, floa
   b = fmaf(s, b, 0.25366922587909174f);
   b = fmaf(s, b, -1.2337005425945717f);
   b = fmaf(s, b, 1.0f);
-  const unsigned q = (unsigned)(int)n;
+  const unsigned q = (unsigned)__double2loint(sum);
   const float x = (q & 1u) ? a : b, y = (q & 1u) ? b : a;
   cn = __uint_as_float(__float_as_uint(x) ^ (((q + 1u) & 2u) << 30));
   sn = __uint_as_float(__float_as_uint(y) ^ ((q & 2u) << 30));
@@ -1201,11 +1198,11 @@ __device__ __forceinline__ void pair_sr(const DirectDev &p, Real rx, Real ry, Re
   } else {
     (void)topA;
     (void)topB;
-    // exp(i k0 r)/r; FP64: the phase k0r r reduced modulo 2 pi first
+    // exp(i k0 r)/r, the phase k0r r reduced in FP64
     Real r, ri, sn, cn;
     if constexpr (sizeof(Real) == 4) {
       inv_and_root(r2, ri, r);
-      phase_sincos(r, p.k0q[0], p.k0q[1], sn, cn);
+      phase_sincos(r, p.k0q, sn, cn);
     } else {
       r = sqrt(r2);
       ri = (Real)1 / r;

@@ -1,7 +1,8 @@
 """The FP32 pair functions that replace library calls (mixed precision):
 r^alpha with 2 alpha an integer (roots and products), the ones beside them
-that still call pow, and Helmholtz with and without damping, phases up to a turn, in the neighbour-list walk and the cell rows, against the
-oracle on the same grid.
+that still call pow, and Helmholtz with and without damping, phases up to
+three turns, in the neighbour-list walk and the cell rows, against the oracle
+on the same grid or against FP64.
 
 Bound: each FP32 pair term is within a few 6e-8 of its value; the sums of a
 few hundred terms of either sign stay within 1e-6 of V and 1e-5 of the
@@ -99,3 +100,52 @@ def test_ralpha_coincident_charges(alpha, side):
         assert np.array_equal(a[at, 0], b[at, 0]) and np.isinf(a[at, 0]).all(), (a[at, 0], b[at, 0])
     assert np.sqrt(np.mean((a[far, 0] - c[far, 0]) ** 2)) < 1e-6 * rms
     assert np.sqrt(np.mean((a[far, 1:] - c[far, 1:]) ** 2)) < 5e-6 * np.sqrt(np.mean(c[far, 1:] ** 2))
+
+
+@pytest.mark.parametrize("lists", ["on", "off"])
+@pytest.mark.parametrize("kw", [dict(alpha=a) for a in (0.5, 1.0, 2.5, 3.0, -0.5, -3.0, 0.3)] +
+                         [dict(k0_r=k, k0_i=0.0) for k in (0.3, 1.0, 2.0, 3.0)] + [dict(k0_r=0.5, k0_i=0.1)])
+def test_one_source(kw, lists):
+    """One unit source, every target inside the cutoff: V is the pair function
+    itself, mixed against FP64, phases to three turns.  Bound: the short-range
+    part is the kernel less its matched polynomial, each rounded to FP32 a few
+    times, so a few 6e-8 of S = |f| + sum |a_k| r^2k at the cutoff (for k0 = 3
+    that sum is 1e3 times the kernel: hence the wide bounds of large phases),
+    and for the grid part 1e-6 of the largest |V|, or for growing kernels 4e-7
+    of the kernel across the grid's box, edges 2 (4 + 8): the FP32 transforms
+    round by that scale (r^3: 9e3, where the pair itself is at most 216)."""
+    import ctypes as C
+    import npme_amd as N
+    print("case one source", kw, lists, flush=True)
+    cx = "k0_r" in kw
+    kind, Rdir, Nder = ("Helmholtz" if cx else "Ralpha"), 6.0, 6
+    rng = np.random.default_rng(4)
+    coord = 4.0 + rng.uniform(-3.4, 3.4, (3000, 3))
+    coord[0] = 4.0
+    r = np.linalg.norm(coord - coord[0], axis=1)
+    q = np.zeros(len(r), complex if cx else float)
+    q[0] = 1.0
+    V = {}
+    for prec in ("mixed", "fp64"):
+        k = N.NPME_KeywordInput(calcType="pme", funcType=kind, EwaldSplit="DerivMatch", Rdir=Rdir, BnOrder=6, tol=1e-6,
+                                precision=prec, N1=64, N2=64, N3=64, n1=16, n2=16, n3=16, nDeriv=Nder,
+                                neighborList=lists, **kw)
+        assert N.NPME_AddMissingKeywords(k, len(q), coord, **({"chargeComplex": q} if cx else {"chargeReal": q}))
+        h = (N.NPME_Interface_SetUpComplexKernel if cx else N.NPME_Interface_SetUpRealKernel)(k, len(q), coord)
+        assert h is not None, N.npme_last_error()
+        V[prec] = h.calcv(q)
+    a, b = np.zeros((Nder + 1, 2)), np.zeros((Nder + 1, 2))
+    assert N.lib().npme_dm_coefficients(kind.encode(), C.c_double(kw.get("alpha", 0.0)), C.c_double(kw.get("k0_r", 0.0)),
+                                        C.c_double(kw.get("k0_i", 0.0)), C.c_int(Nder), C.c_double(Rdir),
+                                        a.ctypes.data_as(C.c_void_p), b.ctypes.data_as(C.c_void_p)) == 0
+    R2k = Rdir ** (2.0 * np.arange(Nder + 1))
+    at = (r > 0.3) & (r < Rdir)
+    f = np.abs(V["fp64"][at])
+    S = [f[:, 0].max() + np.sum(np.hypot(*a.T) * R2k), f[:, 1:].max() + Rdir * np.sum(np.hypot(*b.T) * R2k)]
+    d = np.abs(V["mixed"] - V["fp64"])[at]
+    err = [d[:, 0].max(), d[:, 1:].max()]
+    print("V %.2e of S, %.2e of max; gradient %.2e, %.2e" % (err[0] / S[0], err[0] / f[:, 0].max(), err[1] / S[1],
+                                                             err[1] / f[:, 1:].max()))
+    across = (12.0 * np.sqrt(3.0)) ** kw.get("alpha", -1.0)
+    grid = [max(1e-6 * f[:, 0].max(), 4e-7 * across), max(1e-6 * f[:, 1:].max(), 4e-7 * across)]
+    assert err[0] < 2.4e-7 * S[0] + grid[0] and err[1] < 2.4e-7 * S[1] + grid[1], (err, S, grid)
