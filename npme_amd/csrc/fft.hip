@@ -271,7 +271,12 @@ template <typename T, int A, int B> __device__ __forceinline__ void dft_coprime(
 template <int R, int I> struct TwConst {
   static constexpr double c = ct_cos(I, R), s = ct_sin(I, R);
 };
-// x * exp(-2 pi i I / R)
+// x * exp(-2 pi i I / R).  FP32: the low part of a constant is added where it
+// exceeds 1e-8.  A rounded constant scales every element it meets alike, so
+// its error does not average out as a table's does: with cos(pi/8) off by
+// 2.8e-8, V's error on grids with a radix 16 stage was 2 to 8% above that of
+// radices up to 8 (1/r, 200 boxes: 144^3 1.01, 256^3 1.08 of it); with the low
+// parts it is 0.83 and 0.91 of it, for at most 2% of those passes' time.
 template <typename T, int R, int I> __device__ __forceinline__ T mul_root(T x)
 {
   using S = decltype(T::x);
@@ -279,6 +284,22 @@ template <typename T, int R, int I> __device__ __forceinline__ T mul_root(T x)
   else if constexpr (4 * (I % R) == R) return mul_mi(x);
   else {
     constexpr S c = (S)TwConst<R, I>::c, s = (S)TwConst<R, I>::s;
+    if constexpr (sizeof(S) == 4) {
+      constexpr S dc = (S)(TwConst<R, I>::c - (double)c), ds = (S)(TwConst<R, I>::s - (double)s);
+      constexpr bool lc = dc > 1e-8f || dc < -1e-8f, ls = ds > 1e-8f || ds < -1e-8f;
+      S re = x.y * s, im = -x.x * s;
+      if constexpr (lc && ls) {
+        re = fmaf(x.y, s, fmaf(x.x, dc, x.y * ds));
+        im = fmaf(-x.x, s, fmaf(x.y, dc, -x.x * ds));
+      } else if constexpr (lc) {
+        re = fmaf(x.y, s, x.x * dc);
+        im = fmaf(-x.x, s, x.y * dc);
+      } else if constexpr (ls) {
+        re = fmaf(x.y, s, x.y * ds);
+        im = fmaf(-x.x, s, -x.x * ds);
+      }
+      return mk<T>(fmaf(x.x, c, re), fmaf(x.y, c, im));
+    }
     return mk<T>(x.x * c + x.y * s, x.y * c - x.x * s);
   }
 }
