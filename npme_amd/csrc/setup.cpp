@@ -508,7 +508,7 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   DevBuf srcS, resS;  // sorted order, moved to the fine order below
   if (h.useFine) {
     srcS.reset(4 * rs * (n + 1));
-    resS.reset(sizeof(float4) * (n + 1));
+    if (!f64) resS.reset(sizeof(float4) * (n + 1));
   }
   geometry_charges_device(g, f64, n, h.d_coordS, h.d_perm, h.d_cell, h.useFine ? srcS.p : h.d_src,
                           h.useFine ? resS.p : h.d_srcRes, h.d_ms,
@@ -1124,7 +1124,11 @@ void handle_setup(Handle &h, const Keywords &kw, size_t n, const double *coord)
     else if (b > N / 4) os << "block size n" << d + 1 << " = " << b << " > N/4";
     else if (b < 1 || N % (2 * b) != 0) os << "N" << d + 1 << " must be a multiple of 2 n" << d + 1;
     if (!os.str().empty()) throw Error{NPME_ERR_GRID, os.str()};
-    if (make_plan((int)N).nst < 0) throw Error{NPME_ERR_GRID, "FFT size has a prime factor > 7"};
+    // (every such length up to 4095 has a plan; longer ones are refused below)
+    long rest = N;
+    for (long f : {2, 3, 5, 7})
+      while (rest % f == 0) rest /= f;
+    if (rest != 1) throw Error{NPME_ERR_GRID, "FFT size has a prime factor > 7"};
     h.M[d] = N / 2;
   }
   if (h.Bn < 2 || h.Bn > 16) throw Error{NPME_ERR_UNSUPPORTED, "BnOrder must be in [2, 16]"};

@@ -227,3 +227,34 @@ def test_bench_stall_watch():
     time.sleep(0.6)
     w.stop()
     assert len(fired) == 1
+
+
+def test_fft_plans():
+    """Every length that the grid rules admit (multiples of 4 to 4092 with
+    factors 2, 3, 5, 7) has a plan of 2 to 4 radices that the kernels provide,
+    an even one first, and no stage has more butterflies than the stages'
+    index arithmetic allows (j Ns < 2^22)."""
+    import npme_amd
+    L = ctypes.CDLL(npme_amd.LIB_PATH)
+    make_plan = L._ZN4npme9make_planEi
+    make_plan.argtypes, make_plan.restype = [ctypes.c_void_p, ctypes.c_int], None  # result by hidden pointer
+    used = set()
+    for N in range(8, 4096, 4):
+        rest = N
+        for f in (2, 3, 5, 7):
+            while rest % f == 0:
+                rest //= f
+        plan = (ctypes.c_int * 26)()
+        make_plan(plan, N)
+        radix = list(plan[2:2 + max(plan[1], 0)])
+        if rest != 1:
+            assert plan[1] == -1, N
+            continue
+        assert plan[0] == N and 2 <= len(radix) <= 4 and np.prod(radix) == N and radix[0] % 2 == 0, (N, radix)
+        for order in (radix, radix[::-1]):
+            Ns = 1
+            for R in order:
+                assert (N // R) * Ns < 1 << 22, (N, radix)
+                Ns *= R
+        used |= set(radix)
+    assert used == {2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 16}, used

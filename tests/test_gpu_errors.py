@@ -85,3 +85,15 @@ def test_reset_coord_out_of_memory_leaves_no_state():
     assert not h.CalcV(V, len(q), q, coord) and "no valid set-up" in N.npme_last_error()
     assert h.ResetCoord(len(q), coord)
     assert np.array_equal(h.calcv(q), V0)
+
+
+@pytest.mark.parametrize("n,reason", [(7500, "above 4095"), (4400, "prime factor"), (1100, "prime factor")])
+def test_refused_lengths_name_the_reason(n, reason):
+    """7500 = 2^2 3 5^4 has small factors, and no plan: it is too long."""
+    import npme_amd as N
+    coord, q = uniform_box(300, 20.0)
+    k = N.NPME_KeywordInput(calcType="pme", funcType="Laplace", Rdir=6.0, BnOrder=6, tol=1e-6, nDeriv=6,
+                            EwaldSplit="DerivMatch", N1=36, N2=36, N3=n, n1=9, n2=9, n3=n // 4)
+    N.NPME_AddMissingKeywords(k, len(q), coord, chargeReal=q)
+    assert N.NPME_Interface_SetUpRealKernel(k, len(q), coord) is None
+    assert reason in N.npme_last_error(), N.npme_last_error()
