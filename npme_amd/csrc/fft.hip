@@ -74,17 +74,6 @@ template <typename T> __device__ __forceinline__ T load_or_zero(const T *p, long
   const T x = p[ok ? idx : 0];
   return ok ? x : mk<T>(0, 0);
 }
-__device__ __forceinline__ float load_or_zero(const float *p, long idx, bool ok)
-{
-  const float x = p[ok ? idx : 0];
-  return ok ? x : 0.f;
-}
-__device__ __forceinline__ double load_or_zero(const double *p, long idx, bool ok)
-{
-  const double x = p[ok ? idx : 0];
-  return ok ? x : 0.0;
-}
-
 constexpr int NT = 256;  // threads per workgroup of the 8^L kernels
 
 // stages of a general plan: radices in forward order; for the forward (F)
@@ -1348,6 +1337,8 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
   const int mode = backward ? PASS_BACK : 2 * g.Lin == g.N && g.Lout == g.N ? PASS_FWD : PASS_WHOLE;
   if (backward && (g.Lin != g.N || 2 * g.Lout != g.N))
     throw Error{NPME_ERR_ARG, "backward pass: all of a column in, half of it out"};
+  // whole transforms are the kernel grid's, in FP64
+  if (mode == PASS_WHOLE && !fp64) throw Error{NPME_ERR_ARG, "whole forward transforms run in FP64"};
   const bool half8 = 2 * g.Lin == g.N, full8 = g.Lin == g.N;
   if (!rows && L8 > 0 && (backward ? full8 && 2 * g.Lout == g.N : (half8 || full8) && g.Lout == g.N)) {
     // N = 8^L: the compile-time kernel (4096 / N columns per workgroup)
@@ -1361,7 +1352,7 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
   do {                                                                                         \
     if (backward) NPME_F8(R, LV, false, true);                                                 \
     else if (half8) NPME_F8(R, LV, true, false);                                               \
-    else NPME_F8(R, LV, false, false);                                                         \
+    else if constexpr (sizeof(R) == 8) NPME_F8(R, LV, false, false);                           \
   } while (0)
     if (fp64) {
       if (L8 == 2) NPME_F8L(double, 2);
@@ -1394,7 +1385,7 @@ void fft_pass_complex(bool fp64, const PassGeom &g, const FFTPlan1D &plan, const
   do {                                                                                         \
     if (mode == PASS_FWD) NPME_FFTC(R, PASS_FWD);                                              \
     else if (mode == PASS_BACK) NPME_FFTC(R, PASS_BACK);                                       \
-    else NPME_FFTC(R, PASS_WHOLE);                                                             \
+    else if constexpr (sizeof(R) == 8) NPME_FFTC(R, PASS_WHOLE);                               \
   } while (0)
   if (fp64) NPME_FFTM(double);
   else NPME_FFTM(float);

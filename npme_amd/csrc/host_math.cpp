@@ -509,7 +509,6 @@ void Keywords::set(const std::string &k, double v)
 void Keywords::set(const std::string &k, long v) { set(k, std::to_string(v)); }
 
 // ---------------------------------------------------------------- FFT plan
-// radices 8, 4, 2, 7, 5, 3 (largest first)
 // radices of a length-N transform, largest first after an even first one
 // (the passes prune the zero half of a column in the first stage, whose
 // radix must be even): of all factorisations of N into the butterflies the
