@@ -1,6 +1,7 @@
 """The direct sum of densely packed charges (blocks of 64 targets and groups
 of 16 sources of one cell, k_direct_fine) against the oracle and against the
-cell-row walk (host set-up), for every kernel in both precisions: packed balls
+cell-row walk (which the host set-up takes), for every kernel in both
+precisions: packed balls
 with cells of hundreds of charges, partial blocks and groups, stray charges
 alone in their cells, near-coincident pairs (the fixed point's residuals), a
 cluster of one cell per axis and stencils of nNeigh 1 to 3.
@@ -69,3 +70,47 @@ def test_dense_cells(oracle, nNeigh, nClust, kind, kw, prec):
     # round by 1.8e-15 in the two frames, 2e-12 of that distance: three such
     # charges of 8009 add 2e-6 sqrt(3 / 8009) to a mean gradient of 35, 1e-9
     assert m["relV"] < 1e-11 and m["reldV"] < 1e-9, m
+
+
+@pytest.mark.parametrize("kind,kw", [("Laplace", {}), ("Ralpha", {"alpha": -1.5}),
+                                     ("Helmholtz", {"k0_r": 0.5, "k0_i": 0.0}),
+                                     ("Helmholtz", {"k0_r": 0.5, "k0_i": 0.1})])
+def test_dense_cells_mixed_against_oracle(oracle, kind, kw):
+    """Mixed V within 1e-6 of the oracle, the gradients within 1e-5; those of
+    the charges 1e-3 apart (up to 1e6 where the others have about 35) on
+    their own, within 1e-5 of themselves."""
+    print("case dense cells mixed", kind, kw, flush=True)
+    cx = kind == "Helmholtz"
+    coord, q = _charges(8009, cx)
+    h = _setup(kind, "mixed", coord, q, "device", 2, 3, **kw)
+    assert "dense cells" in h.Print()
+    V = h.calcv(q)
+    ok = {"Laplace": lambda: oracle.kernel(oracle.LAPLACE, 6, 4.0),
+          "Ralpha": lambda: oracle.kernel(oracle.RALPHA, 6, 4.0, alpha=kw.get("alpha", 0.0)),
+          "Helmholtz": lambda: oracle.kernel(oracle.HELMHOLTZ, 6, 4.0,
+                                             k0=complex(kw.get("k0_r", 0.0), kw.get("k0_i", 0.0)))}[kind]()
+    Vo = oracle.calcv(ok, (96, 96, 96), 6, coord, q)
+    close = np.r_[20:23, 30:33]
+    far = np.setdiff1d(np.arange(len(q)), close)
+    rms = lambda x: np.sqrt(np.mean(np.abs(x) ** 2))
+    err = [rms(V[far, 0] - Vo[far, 0]) / rms(Vo[far, 0]), rms(V[far, 1:] - Vo[far, 1:]) / rms(Vo[far, 1:]),
+           rms(V[close] - Vo[close]) / rms(Vo[close])]
+    print(err)
+    assert err[0] < 1e-6 and err[1] < 1e-5 and err[2] < 1e-5, err
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_dense_sparse_dense(prec):
+    """ResetCoord from dense cells to sparse ones and back: direct sum, order
+    and graph are those of a fresh handle, bit for bit."""
+    print("case dense sparse dense", prec, flush=True)
+    dense, q = _charges(8009, False)
+    sparse = uniform_box(8009, 36.0)[0]
+    h = _setup("Laplace", prec, dense, q, "device", 2, 3)
+    for coord, name in ((dense, "dense cells"), (sparse, "cell rows"), (dense, "dense cells")):
+        assert h.ResetCoord(len(q), coord)
+        fresh = _setup("Laplace", prec, coord, q, "device", 2, 3)
+        assert name in h.Print() and name in fresh.Print()
+        V = fresh.calcv(q)
+        for _ in range(3):  # launched, captured, replayed
+            assert np.array_equal(h.calcv(q), V)

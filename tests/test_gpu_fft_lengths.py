@@ -1,5 +1,6 @@
-"""The general FFT passes at lengths that use every radix (2 to 10, 12, 16)
-and two, three and four stages, on each of the three axes: CalcV on a given
+"""The general FFT passes at lengths that use every radix (2 to 10, 12, 16;
+2 only at 8 to 32) and two, three and four stages, to the longest lengths
+(4092 at most), on each of the three axes: CalcV on a given
 grid against the oracle on the same grid.  Real charges (R2C and C2R rows,
 columns, convolution) and complex ones (complex rows), FP64 and mixed.
 
@@ -20,9 +21,17 @@ GRIDS = [(36, 40, 48), (64, 56, 60), (100, 108, 112), (144, 140, 160), (280, 36,
          (36, 540, 40), (40, 36, 500), (980, 36, 40), (36, 1372, 40), (40, 36, 1260)]
 
 
-def _setup(kind, prec, grid, coord):
+# with a spline of order 4: 20 = 10 2, 24 = 12 2, 32 = 16 2
+SHORT = [(20, 24, 32), (32, 20, 24), (24, 32, 20)]
+# one column to a workgroup in FP64 (rows of more than half its LDS), the
+# largest workgroups and index quotients: 3840 = 10 8 8 6, 4032 = 8 9 8 7,
+# 4000 = 10 10 8 5, 2592 = 8 9 6 6, 3888 = 8 9 9 6
+LONG = [(36, 40, 3840), (4032, 36, 40), (36, 4000, 40), (2592, 36, 40), (40, 3888, 36), (36, 40, 4032)]
+
+
+def _setup(kind, prec, grid, coord, Bn=6):
     import npme_amd as N
-    kw = dict(calcType="pme", EwaldSplit="DerivMatch", Rdir=6.0, BnOrder=6, tol=1e-6, precision=prec,
+    kw = dict(calcType="pme", EwaldSplit="DerivMatch", Rdir=6.0, BnOrder=Bn, tol=1e-6, precision=prec,
               nDeriv=6, fftKernels="generic")
     kw.update({"N%d" % (d + 1): n for d, n in enumerate(grid)})
     kw.update({"n%d" % (d + 1): n // 4 for d, n in enumerate(grid)})
@@ -50,6 +59,27 @@ def test_fft_lengths_match_oracle(oracle, grid, kind, prec):
     k = oracle.kernel(oracle.LAPLACE, 6, 6.0) if kind == "Laplace" else \
         oracle.kernel(oracle.HELMHOLTZ, 6, 6.0, k0=0.5)
     m = oracle.compare_v(oracle.calcv(k, grid, 6, coord, q), V)
+    print(m["relV"], m["reldV"])
+    bound = (1e-11, 1e-11) if prec == "fp64" else (1e-6, 1e-5)
+    assert m["relV"] < bound[0] and m["reldV"] < bound[1], m
+
+
+def _cases():
+    return [(g, 4) for g in SHORT] + [(g, 6) for g in LONG]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["Laplace", "Helmholtz"])
+@pytest.mark.parametrize("grid,Bn", _cases())
+def test_fft_shortest_and_longest_lengths(oracle, grid, Bn, kind, prec):
+    print("case fft lengths", grid, Bn, kind, prec, flush=True)
+    coord, q = uniform_box(401, 20.0)
+    if kind == "Helmholtz":
+        q = q + 1j * uniform_box(401, 20.0, 7, 8)[1]
+    V = _setup(kind, prec, grid, coord, Bn).calcv(q)
+    k = oracle.kernel(oracle.LAPLACE, 6, 6.0) if kind == "Laplace" else \
+        oracle.kernel(oracle.HELMHOLTZ, 6, 6.0, k0=0.5)
+    m = oracle.compare_v(oracle.calcv(k, grid, Bn, coord, q), V)
     print(m["relV"], m["reldV"])
     bound = (1e-11, 1e-11) if prec == "fp64" else (1e-6, 1e-5)
     assert m["relV"] < bound[0] and m["reldV"] < bound[1], m
