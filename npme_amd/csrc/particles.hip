@@ -2564,14 +2564,21 @@ __global__ __launch_bounds__(64 * W) void k_spread_mfma64(int BnRun, long M1, lo
 // charges, ~8 us each (dependent loads, FP64 spline weights, LDS staging,
 // products), so with few tiles a launch is as long as its longest chain of
 // chunks: 22k charges on 96^3 (108 tiles of ~11 chunks) 76 -> 26 us, 1k charges
-// on 48^3 (18 tiles) 41 -> 15 us with several wavefronts a tile.  With
-// enough tiles one wavefront is best (the sums across wavefronts are extra):
-// the chip holds 4 wavefronts on each of its 1024 SIMDs.
-static int spread_waves(long tiles, size_t entries)
+// on 48^3 (18 tiles) 41 -> 15 us with several wavefronts a tile.  (The chain is
+// judged by the mean tile: packed sets get the wavefronts of their tile
+// count, 300 -> 83 us for 6k charges in a ball on 64^3.)
+// With enough tiles one wavefront is best, the sums across wavefronts being
+// extra.  The line is where the chip is full: 4 wavefronts on each of 1024
+// SIMDs (FP32, 100k charges on 252^3: 4,096 wavefronts 24.8 us against 27.0
+// with half of them, 8,192 on larger grids no gain; complex 192^3 3,456 31.4
+// against 37.0); FP64 real tiles stage 16 KB a wavefront, 10 to a CU, 2,560
+// on the chip (224^3: 2,744 wavefronts 30.4 us against 31.7 with half, 240^3:
+// 3,600 31.7 against 27.6).
+static int spread_waves(long tiles, size_t entries, long most)
 {
   const long chunks = (long)((entries + 63) / 64 + tiles - 1) / std::max(tiles, 1L);  // of a mean tile
   int w = 1;
-  while (w < 4 && (long)w * 2 * tiles <= 4096 && 2 * w <= chunks + 1) w *= 2;
+  while (w < 4 && (long)w * 2 * tiles <= most && 2 * w <= chunks + 1) w *= 2;
   return w;
 }
 
@@ -2580,8 +2587,8 @@ void launch_spread(bool fp64, bool complexK, long Bn, const long M[3], const int
                    const void *qim, const int4 *ms, const void *frac, void *grid, hipStream_t s)
 {
   const dim3 g((unsigned)(nt[0] * nt[1] * nt[2]));
-  const int W = spread_waves((long)nt[0] * nt[1] * nt[2], entries);
   const bool mfma = !complexK;  // 16 x 8 x 8 tiles on the matrix cores, else 8^3
+  const int W = spread_waves((long)nt[0] * nt[1] * nt[2], entries, fp64 && mfma ? 3072 : 4096);
   if (T[0] != (mfma ? 16 : 8) || T[1] != 8 || T[2] != 8) throw Error{NPME_ERR_UNSUPPORTED, "spreading tile shape"};
 #define NPME_SPREAD_K(KERNEL, R, ...)                                                            \
   hipLaunchKernelGGL(KERNEL, g, dim3(64 * W), 0, s, (int)Bn, M[0], M[1], M[2], nt[0], nt[1], nt[2], \
