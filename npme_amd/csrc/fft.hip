@@ -1259,7 +1259,10 @@ struct FftLaunch {
 // columns: all of it)
 constexpr size_t kFftLds = 80 * 1024, kFftLdsMax = 160 * 1024;
 // a launch should have this many workgroups (four for each of 256 CUs)
-// before workgroups are made wider
+// before workgroups are made wider.  Sum of the passes, us, by lines of 512 /
+// 1,024 / 2,048 / 8,192: 1/r 96^3 39.2 / 40.5 / 40.4 / 40.4, 280^3 120.6 / 120.2 /
+// 124.8 / 129.1; FP64 96^3 42.6 / 45.7 / 45.7 / 45.6, 360^3 410 / 410 / 408 / 434
+// (small grids would take 512, large ones lose from 2,048 on)
 constexpr long kFftWide = 1024;
 
 // strided columns: 16 adjacent columns for short lengths where there are

@@ -98,7 +98,9 @@ __device__ __forceinline__ size_t lower_bound_d(const K *a, size_t n, K v)
 // of a merge sort (600k charges: 260 us, launches of ~6 us with ~5 us between
 // them).  Ranking is quadratic in a cell, so cells of more than kRankMax
 // charges raise GEO_LONG_BUCKET and the phase is repeated with the radix
-// sort.
+// sort.  Set-up of 1M charges, ranked against sorted (the pass up to the
+// ranking included): 1,000 a cell 1.83 / 1.98 ms, 2,000 2.12 / 2.17, 4,000
+// 2.36 / 2.23; 300k: 0.86 / 0.98, 0.92 / 0.99, 0.98 / 1.00.
 constexpr int kRankMax = 2048;
 
 __global__ __launch_bounds__(256) void k_cell_place(size_t n, const unsigned *__restrict__ key,
@@ -604,7 +606,10 @@ void geometry_cells_device(const GeoParams &g, size_t n, const double *d_coord, 
 // time, and ~32 opened chunks) are scanned, larger sets sorted: the scan costs
 // ~25 instructions a step, twice; the radix sort of 22k charges' 77k entries
 // takes 10 launches (100 us; the scan 30 us), that of 600k charges' 2.1M entries
-// 120 us
+// 120 us.  Whole set-ups, scanned / sorted, by work: 5.7e5 (1M on 256^3) 12.43 /
+// 12.59 ms, 6.7e5 (300k on 360^3) 7.00 / 7.03, 9.2e5 (100k on 512^3) 3.71 / 3.67,
+// 1.7e6 (300k on 512^3) 7.61 / 7.39, 4.5e6 (1M on 512^3) 14.2 / 13.0; packed sets
+// may lose below the line as well (600k in a ball on 256^3, 3.7e5: 1.49 / 1.40)
 constexpr double kScanWork = 1.0e6;
 static bool scan_tiles(long nt, size_t n) { return (double)nt * ((double)n / 4096.0 + 32.0) <= kScanWork; }
 

@@ -463,7 +463,12 @@ static bool particles_device(Handle &h, GeoParams &g, const std::string &nlmode,
   // without a list: the fine order when the blocks of 64 charges of one cell
   // are at least half full on average (sparser cells leave its lanes idle,
   // where the cell rows' blocks of 8 do not) and the stencil's differences fit
-  // the list's frame, else the cell rows
+  // the list's frame, else the cell rows.  Direct sum of 100k charges, fine
+  // order against cell rows, us: 30 charges a block, nNeigh 2: 1/r 536 / 1541,
+  // FP64 825 / 1576, Helmholtz 1048 / 1831; nNeigh 3: 1190 / 2249, 1892 / 2426,
+  // 2523 / 2912 (and at 31 a block 2808 / 2763); 6 a block: nNeigh 2 695 / 1062,
+  // 1143 / 1019, 1241 / 1198, nNeigh 3 FP64 1759 / 1474.  So the line is where no
+  // kernel loses; 1/r alone would gain from 6 on
   if (!list && !h.trans && !kind_ref_pairs(h.ker.kind) && h.nNeigh <= 3 && h.nNeigh + 1 < 2 * h.nCellClust1D) {
     DevBuf start;
     const int nb = fine_blocks_device(g, h.d_cellStart, start, s);
@@ -1248,7 +1253,9 @@ void handle_setup(Handle &h, const Keywords &kw, size_t n, const double *coord)
     };
     // grids with few tiles take smaller ones, down to edge 4, until every CU
     // has one: a launch of 27 workgroups is as long as one of them (96^3
-    // grid, 22k charges: 27 tiles of edge 16 30 us, 216 of edge 8 10 us)
+    // grid, 22k charges: 27 tiles of edge 16 30 us, 216 of edge 8 10 us).  Any
+    // line from 128 to 512 tiles is as good (5k to 100k charges, within 2%),
+    // 1,024 is not (60k FP64 19.4 -> 27.3 us: the halo grows)
     const int edges[] = {16, 12, 8, 6, 4, 2, 1};
     for (int e : edges) {
       h.TI = e;
