@@ -8,10 +8,11 @@ Bound: each FP32 pair term is within a few 6e-8 of its value; the sums of a
 few hundred terms of either sign stay within 1e-6 of V and 1e-5 of the
 gradient, the bounds of the mixed form elsewhere.  For r^3 the smooth part
 dwarfs the pair terms and V's error is the FP32 grid's, which changes several
-times over with the box alone (2.0e-7 to 5.9e-7 over six boxes at 64^3; the
-box used here is above 1e-6), so its bound is on the geometric mean over boxes.
-Wave numbers beyond a turn inside the cutoff are left out: the matched
-polynomials cancel there.  (k0 = 2 has the same error as with library sines.)"""
+times over with the box alone (2.0e-7 to 6.7e-7 over the boxes here at 64^3), so
+its bound is on the geometric mean over boxes, and a wider one on each.
+Against the oracle wave numbers stay below a turn inside the cutoff, since the
+matched polynomials cancel beyond; one source alone is taken to three turns.
+(k0 = 2 has the same error as with library sines.)"""
 import numpy as np
 import pytest
 
@@ -149,3 +150,26 @@ def test_one_source(kw, lists):
     across = (12.0 * np.sqrt(3.0)) ** kw.get("alpha", -1.0)
     grid = [max(1e-6 * f[:, 0].max(), 4e-7 * across), max(1e-6 * f[:, 1:].max(), 4e-7 * across)]
     assert err[0] < 2.4e-7 * S[0] + grid[0] and err[1] < 2.4e-7 * S[1] + grid[1], (err, S, grid)
+
+
+def test_ralpha_cubed_each_box():
+    """r^3 box by box, against FP64 on the same grid: V within 2.4e-6, five
+    times the rms of 300 boxes at 64^3 (4.8e-7; most of it the grid's k = 0
+    term, a shift of V that is Gaussian over boxes), and without the shift
+    within 1.4e-6, five times 2.8e-7."""
+    import npme_amd as N
+    for seed, L in ((0, 20.0), (1, 27.3), (5, 30.0), (9, 31.7), (13, 34.1), (21, 41.3)):
+        print("case r^3 box", seed, L, flush=True)
+        coord, q = uniform_box(1500, L, seed, seed + 1) if seed else uniform_box(1500, L)
+        V = {}
+        for prec in ("mixed", "fp64"):
+            k = N.NPME_KeywordInput(calcType="pme", funcType="Ralpha", EwaldSplit="DerivMatch", Rdir=6.0, BnOrder=6,
+                                    tol=1e-6, precision=prec, N1=64, N2=64, N3=64, n1=16, n2=16, n3=16, nDeriv=6,
+                                    alpha=3.0)
+            assert N.NPME_AddMissingKeywords(k, len(q), coord, chargeReal=q), N.npme_last_error()
+            h = N.NPME_Interface_SetUpRealKernel(k, len(q), coord)
+            assert h is not None, N.npme_last_error()
+            V[prec] = h.calcv(q)[:, 0]
+        d, norm = V["mixed"] - V["fp64"], np.linalg.norm(V["fp64"])
+        print("%.2e %.2e" % (np.linalg.norm(d) / norm, np.linalg.norm(d - d.mean()) / norm))
+        assert np.linalg.norm(d) < 2.4e-6 * norm and np.linalg.norm(d - d.mean()) < 1.4e-6 * norm
